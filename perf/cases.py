@@ -463,6 +463,24 @@ def _exact_adjoint(case, seed):
     return {k: torch.stack(v).cpu().numpy() for k, v in zip(("action", "grad", "params", "energy"), zip(*out))}
 
 
+def _bessel(z):
+    """J0 and Y0 in FP64 (torch's are good to about 1e-7): the power series below 2, above it the integral
+    H0(z) = sqrt(2 / z) / pi e^{i (z - pi / 4)} int exp(-t^2) (1 + i t^2 / 2z)^{-1/2} dt, which the trapezoid rule
+    takes to full precision."""
+    low = z < 2.0
+    s, t, js, ys, harm = torch.where(low, z, 1.0), 1.0, 1.0, 0.0, 0.0
+    for k in range(1, 20):
+        t, harm = t * (-0.25 * s * s / (k * k)), harm + 1.0 / k
+        js, ys = js + t, ys - t * harm
+    ys = (2.0 / math.pi) * ((torch.log(0.5 * s) + 0.57721566490153286061) * js + ys)
+    b, total, step = torch.where(low, 2.0, z), 0.0, 0.125
+    for i in range(-52, 53):
+        u = (i * step) ** 2
+        total = total + math.exp(-u) * torch.rsqrt(torch.complex(torch.ones_like(b), 0.5 * u / b))
+    hankel = torch.sqrt(2.0 / b) * (step / math.pi) * total * torch.exp(1j * (b - 0.25 * math.pi))
+    return torch.where(low, js, hankel.real), torch.where(low, ys, hankel.imag)
+
+
 def _exact_table(case, seed):
     """The three Bessel integrals of the pair-product propagator (src/propagator.jl:36-70 of the reference) by
     Gauss-Legendre panels: in log k towards 0, uniform up to where the Gaussian is below 1e-18."""
@@ -480,7 +498,7 @@ def _exact_table(case, seed):
     dev = "cuda" if torch.cuda.is_available() else "cpu"
     r = 1e-20 + torch.arange(case["n"], device=dev, dtype=torch.float64) * ((case["r1"] - 1e-20) / (case["n"] - 1))
     z = r[:, None] * torch.as_tensor(k, device=dev)
-    J, Y = torch.special.bessel_j0(z), torch.special.bessel_y0(z)
+    J, Y = _bessel(z)
     a, b = torch.as_tensor(c, device=dev), torch.as_tensor(c * d, device=dev)
     cross = (J * b) @ Y.T
     return ((Y * a) @ Y.T - (J * a) @ J.T - cross - cross.T).cpu().numpy()
