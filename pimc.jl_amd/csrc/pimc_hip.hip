@@ -183,8 +183,15 @@ struct pimc_ctx {
     int *d_cell_cnt = nullptr, *d_bins = nullptr;
     unsigned short *d_cell_mem = nullptr;
     int *d_status = nullptr;
-    double *d_work = nullptr, *d_io = nullptr;
+    double *d_work = nullptr, *d_io = nullptr, *d_hpart = nullptr;
     size_t work_elems = 0, io_elems = 0;
+    // Pinned host buffer of the single calls: small inputs and results pass through it without a copy
+    // command (the kernels read and write it), larger results by one asynchronous copy, so a call is
+    // one launch and one synchronisation.  Copies larger than kPinBytes go in pieces.
+    unsigned char *h_pin = nullptr;
+    size_t pin_bytes = 0;
+    unsigned long long *d_dens = nullptr; // counts of pimc_density, up to kScratchBins bins
+    std::vector<long long> hcnt; // host copy of the counters after the last run (empty: not known)
     std::vector<Launch> events;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     long long cart_per_chain = 0;
@@ -374,25 +381,12 @@ bool grow_blocks(pimc_ctx *c, int need)
     return true;
 }
 
-// Block b of one chain from the host copy, refreshed after each run.
 // Host to device, ordered on the library stream: that stream is non-blocking, so a plain
 // hipMemcpy (null stream) is not ordered before its kernels.  Returns when the copy is complete.
 void h2d(pimc_ctx *c, void *dst, const void *src, size_t bytes)
 {
     HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-}
-
-const double *host_block(pimc_ctx *c, int b, int chain)
-{
-    if (c->hblk_n != c->nblk) {
-        HIPCHK(hipStreamSynchronize(c->stream));
-        c->hblocks.resize((size_t)c->nblk * c->n_chains * kNQ);
-        if (c->nblk > 0)
-            HIPCHK(hipMemcpy(c->hblocks.data(), c->d_blocks, sizeof(double) * c->hblocks.size(), hipMemcpyDeviceToHost));
-        c->hblk_n = c->nblk;
-    }
-    return &c->hblocks[((size_t)b * c->n_chains + chain) * kNQ];
 }
 
 int check_chain(pimc_ctx *c, int chain)
@@ -414,23 +408,77 @@ int check_table(pimc_ctx *c, int chain)
 }
 
 // Cell-list overflow flags are per chain and stay set until the chain's paths are set again.
+int status_error(pimc_ctx *c, int chain)
+{
+    return set_err(c, PIMC_ERR_CAPACITY, "chain " + std::to_string(chain) +
+                                             ": a cell list overflowed its capacity; raise r_a or lower the density");
+}
+
 int check_status(pimc_ctx *c)
 {
     std::vector<int> st(c->n_chains);
     HIPCHK(hipMemcpy(st.data(), c->d_status, sizeof(int) * c->n_chains, hipMemcpyDeviceToHost));
     for (int i = 0; i < c->n_chains; ++i)
-        if (st[i])
-            return set_err(c, PIMC_ERR_CAPACITY, "chain " + std::to_string(i) +
-                                                     ": a cell list overflowed its capacity; raise r_a or lower the density");
+        if (st[i]) return status_error(c, i);
     return PIMC_OK;
 }
 
-void ensure_io(pimc_ctx *c, size_t n)
+template <typename T> void grow_device(T *&p, size_t &have, size_t n)
 {
-    if (n <= c->io_elems) return;
-    dfree(c->d_io);
-    c->d_io = dalloc<double>(n);
-    c->io_elems = n;
+    if (n <= have) return;
+    dfree(p);
+    p = nullptr;
+    have = 0;
+    p = dalloc<T>(n);
+    have = n;
+}
+
+void ensure_io(pimc_ctx *c, size_t n) { grow_device(c->d_io, c->io_elems, n); }
+
+constexpr size_t kPinBytes = (size_t)4 << 20;
+
+// The context's pinned buffer with room for `bytes`.
+template <typename T> T *pinned(pimc_ctx *c, size_t bytes)
+{
+    if (bytes > c->pin_bytes) {
+        if (c->h_pin) HIPCHK(hipHostFree(c->h_pin));
+        c->h_pin = nullptr;
+        c->pin_bytes = 0;
+        size_t want = 64 * 1024;
+        while (want < bytes) want <<= 1;
+        void *p = nullptr;
+        HIPCHK(hipHostMalloc(&p, want, hipHostMallocDefault));
+        c->h_pin = static_cast<unsigned char *>(p);
+        c->pin_bytes = want;
+    }
+    return reinterpret_cast<T *>(c->h_pin);
+}
+
+// n elements from the device, after the work queued on the library stream: use(p, i0, m) gets the
+// elements i0 .. i0 + m at p, in pieces of the pinned buffer.
+template <typename T, typename Use> void from_device(pimc_ctx *c, const T *src, size_t n, Use use)
+{
+    const size_t per = kPinBytes / sizeof(T);
+    T *const p = pinned<T>(c, std::min(n, per) * sizeof(T));
+    for (size_t i0 = 0; i0 < n; i0 += per) {
+        const size_t m = std::min(per, n - i0);
+        HIPCHK(hipMemcpyAsync(p, src + i0, m * sizeof(T), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        use(p, i0, m);
+    }
+}
+
+// Block b of one chain from the host copy, refreshed after each run.
+const double *host_block(pimc_ctx *c, int b, int chain)
+{
+    if (c->hblk_n != c->nblk) {
+        c->hblocks.resize((size_t)c->nblk * c->n_chains * kNQ);
+        from_device(c, (const double *)c->d_blocks, c->hblocks.size(), [&](const double *p, size_t i0, size_t m) {
+            std::memcpy(c->hblocks.data() + i0, p, m * sizeof(double));
+        });
+        c->hblk_n = c->nblk;
+    }
+    return &c->hblocks[((size_t)b * c->n_chains + chain) * kNQ];
 }
 
 HookArgs hook_args(pimc_ctx *c, int chain)
@@ -443,7 +491,7 @@ HookArgs hook_args(pimc_ctx *c, int chain)
     h.bins = c->d_bins;
     h.status = c->d_status;
     h.chain = chain;
-    h.work = c->d_work;
+    h.n_chains = c->n_chains;
     h.use_cells = (c->ch[chain].ncell > 0) ? 1 : 0;
     h.next = c->d_next + c->ch[chain].part_base;
     return h;
@@ -470,6 +518,16 @@ HookArgs hook_args(pimc_ctx *c, int chain)
         }                                                                                                              \
         HIPCHK(hipGetLastError());                                                                                     \
     } while (0)
+
+// Blocks of the energy and adjoint kernels for one chain: 256 threads each, `lanes` threads per bead,
+// at most kHookMaxBlocks; their partial sums' buffer.
+constexpr int kHookMaxBlocks = 1024;
+int hook_blocks(pimc_ctx *c, int chain, int lanes)
+{
+    if (!c->d_hpart) c->d_hpart = dalloc<double>((size_t)kHookMaxBlocks * kHookSums);
+    const long long n = (long long)c->ch[chain].N * c->ch[chain].M * lanes;
+    return (int)std::max(1LL, std::min<long long>(kHookMaxBlocks, (n + 255) / 256));
+}
 
 // The estimators of one sweep in their own kernels: the whole chains of the
 // wide estimator kernel (k_meas_beads, with or without cell lists) and the
@@ -1465,10 +1523,6 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
         HIPCHK(hipMemset(c->d_rs, 0, sizeof(RunState)));
         c->d_status = dalloc<int>(n_chains);
         HIPCHK(hipMemset(c->d_status, 0, sizeof(int) * n_chains));
-        int maxM = 0;
-        for (int i = 0; i < n_chains; ++i) maxM = std::max(maxM, c->ch[i].M);
-        c->work_elems = (size_t)(maxM + 1) * c->dim + 16;
-        c->d_work = dalloc<double>(c->work_elems);
         if (opt->radial_bins > 0) {
             c->d_radial = dalloc<unsigned long long>((size_t)n_chains * opt->radial_bins);
             HIPCHK(hipMemset(c->d_radial, 0, sizeof(unsigned long long) * n_chains * opt->radial_bins));
@@ -1499,9 +1553,10 @@ int pimc_destroy(pimc_ctx *c)
                     c->d_whole_cells, c->d_whole_brute, c->d_is_whole, c->d_cell_cnt, c->d_bins, c->d_cell_mem,
                     c->d_status, c->d_work, c->d_io, c->d_whole_lds, c->d_next, c->d_meas_ids, c->d_meas_part,
                     c->d_cells_all, c->d_spec, c->d_wbnd, c->d_win_all, c->d_cacc, c->d_cshift, c->d_pm, c->d_win_part,
-                    c->d_beams, c->d_wg_cells[0], c->d_wg_cells[1]};
+                    c->d_beams, c->d_wg_cells[0], c->d_wg_cells[1], c->d_hpart, c->d_dens};
     for (void *p : ptrs) dfree(p);
     for (double *p : c->d_tab) dfree(p);
+    if (c->h_pin) (void)hipHostFree(c->h_pin);
     for (auto &e : c->events) {
         (void)hipEventDestroy(e.a);
         (void)hipEventDestroy(e.b);
@@ -1690,23 +1745,21 @@ int pimc_get_paths(pimc_ctx *c, int32_t chain, double *r)
     const ChainDev &h = c->ch[chain];
     const size_t n = (size_t)h.N * h.dim * h.M;
     try {
-        HIPCHK(hipStreamSynchronize(c->stream));
-        auto src_index = [&](size_t n_, int d_, int j_) -> size_t {
-            return h.sm ? ((size_t)j_ * h.N + n_) * h.dim + d_ : ((size_t)n_ * h.dim + d_) * h.M + j_;
+        // device layout of the chain -> caller layout N x dim x M (Particle.r blocks)
+        auto take = [&](auto *p, size_t i0, size_t m) {
+            if (!h.sm) {
+                for (size_t i = 0; i < m; ++i) r[i0 + i] = p[i];
+                return;
+            }
+            const size_t row = (size_t)h.N * h.dim;
+            size_t j = i0 / row, k = i0 - j * row; // element k = n dim + d of slice j
+            for (size_t i = 0; i < m; ++i) {
+                r[k * h.M + j] = p[i];
+                if (++k == row) k = 0, ++j;
+            }
         };
-        if (c->prec == PIMC_FP64) {
-            std::vector<double> f(n);
-            HIPCHK(hipMemcpy(f.data(), (double *)c->d_pos + h.pos_off, n * sizeof(double), hipMemcpyDeviceToHost));
-            for (int p = 0; p < h.N; ++p)
-                for (int d = 0; d < h.dim; ++d)
-                    for (int j = 0; j < h.M; ++j) r[((size_t)p * h.dim + d) * h.M + j] = f[src_index(p, d, j)];
-        } else {
-            std::vector<float> f(n);
-            HIPCHK(hipMemcpy(f.data(), (float *)c->d_pos + h.pos_off, n * sizeof(float), hipMemcpyDeviceToHost));
-            for (int p = 0; p < h.N; ++p)
-                for (int d = 0; d < h.dim; ++d)
-                    for (int j = 0; j < h.M; ++j) r[((size_t)p * h.dim + d) * h.M + j] = f[src_index(p, d, j)];
-        }
+        if (c->prec == PIMC_FP64) from_device(c, (const double *)c->d_pos + h.pos_off, n, take);
+        else from_device(c, (const float *)c->d_pos + h.pos_off, n, take);
     } catch (const HipError &e) {
         return hip_err(c, e);
     }
@@ -1834,9 +1887,17 @@ int pimc_run(pimc_ctx *c, int32_t n_sweeps, int32_t measure, pimc_counters *out)
         return set_err(c, PIMC_ERR_ARG, "a measuring run must be a multiple of measure_every sweeps");
     if (int rc = check_table(c, -1)) return rc;
     try {
-        std::vector<long long> before((size_t)c->n_chains * kCnt);
-        HIPCHK(hipStreamSynchronize(c->stream));
-        HIPCHK(hipMemcpy(before.data(), c->d_cnt, sizeof(long long) * before.size(), hipMemcpyDeviceToHost));
+        // the counters as the last run left them (they change in runs only); re-read after a failed one
+        const size_t ncnt = (size_t)c->n_chains * kCnt;
+        if (c->hcnt.size() != ncnt) {
+            std::vector<long long> now(ncnt);
+            from_device(c, (const long long *)c->d_cnt, ncnt, [&](const long long *p, size_t i0, size_t m) {
+                std::memcpy(now.data() + i0, p, m * sizeof(long long));
+            });
+            c->hcnt.swap(now);
+        }
+        std::vector<long long> before;
+        before.swap(c->hcnt);
         const int K = c->opt.sweeps_per_launch;
         const int nl = (n_sweeps + K - 1) / K;
         c->hblk_n = -1;
@@ -1876,12 +1937,19 @@ int pimc_run(pimc_ctx *c, int32_t n_sweeps, int32_t measure, pimc_counters *out)
             ++li;
         }
         HIPCHK(hipEventRecord(c->ev1, c->stream));
+        // counters and status words follow the launches: one synchronisation for the run
+        long long *const pin = pinned<long long>(c, ncnt * sizeof(long long) + (size_t)c->n_chains * sizeof(int));
+        const int *const st = reinterpret_cast<const int *>(pin + ncnt);
+        HIPCHK(hipMemcpyAsync(pin, c->d_cnt, ncnt * sizeof(long long), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipMemcpyAsync(pin + ncnt, c->d_status, (size_t)c->n_chains * sizeof(int), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
-        int rc = check_status(c);
+        int rc = PIMC_OK;
+        for (int i = 0; i < c->n_chains && rc == PIMC_OK; ++i)
+            if (st[i]) rc = status_error(c, i);
+        c->hcnt.assign(pin, pin + ncnt);
         if (out) {
             std::memset(out, 0, sizeof(*out));
-            std::vector<long long> after(before.size());
-            HIPCHK(hipMemcpy(after.data(), c->d_cnt, sizeof(long long) * after.size(), hipMemcpyDeviceToHost));
+            const std::vector<long long> &after = c->hcnt;
             for (int i = 0; i < c->n_chains; ++i) {
                 const long long *b = before.data() + (size_t)i * kCnt, *e = after.data() + (size_t)i * kCnt;
                 out->levy_acc += e[0] - b[0];
@@ -1924,8 +1992,8 @@ int pimc_get_counters(pimc_ctx *c, int32_t chain, int64_t *out)
         const int n = (int)c->ch.size();
         const int first = chain < 0 ? 0 : chain, count = chain < 0 ? n : 1;
         std::vector<long long> acc((size_t)count * kCnt);
-        HIPCHK(hipStreamSynchronize(c->stream));
-        HIPCHK(hipMemcpy(acc.data(), c->d_cnt + (size_t)first * kCnt, sizeof(long long) * acc.size(), hipMemcpyDeviceToHost));
+        from_device(c, (const long long *)c->d_cnt + (size_t)first * kCnt, acc.size(),
+                    [&](const long long *p, size_t i0, size_t m) { std::memcpy(acc.data() + i0, p, m * sizeof(long long)); });
         for (int i = 0; i < count; ++i) {
             out[4 * i + 0] = acc[kCnt * i];
             out[4 * i + 1] = acc[kCnt * i + 5];
@@ -1943,7 +2011,6 @@ int pimc_get_blocks(pimc_ctx *c, int32_t chain, double *E, double *Ev, double *E
     int rc = check_chain(c, chain);
     if (rc) return rc;
     try {
-        HIPCHK(hipStreamSynchronize(c->stream));
         std::vector<double> q((size_t)c->nblk * kNQ);
         for (int b = 0; b < c->nblk; ++b)
             std::memcpy(&q[(size_t)b * kNQ], host_block(c, b, chain), sizeof(double) * kNQ);
@@ -1968,7 +2035,6 @@ int pimc_get_estimates(pimc_ctx *c, int32_t chain, pimc_estimates *out)
     if (!out) return set_err(c, PIMC_ERR_ARG, "null output");
     std::memset(out, 0, sizeof(*out));
     try {
-        HIPCHK(hipStreamSynchronize(c->stream));
         const int nb = c->nblk;
         std::vector<double> q((size_t)nb * kNQ);
         for (int b = 0; b < nb; ++b)
@@ -2060,10 +2126,9 @@ int pimc_get_radial(pimc_ctx *c, int32_t chain, double *hist, int64_t *ndata)
     if (!c->d_radial) return set_err(c, PIMC_ERR_STATE, "radial histogram not enabled");
     try {
         const int nb = c->opt.radial_bins;
-        std::vector<unsigned long long> h(nb);
-        HIPCHK(hipStreamSynchronize(c->stream));
-        HIPCHK(hipMemcpy(h.data(), c->d_radial + (size_t)chain * nb, sizeof(unsigned long long) * nb, hipMemcpyDeviceToHost));
-        for (int i = 0; i < nb; ++i) hist[i] = (double)h[i];
+        from_device(c, c->d_radial + (size_t)chain * nb, (size_t)nb, [&](const unsigned long long *h, size_t i0, size_t m) {
+            for (size_t i = 0; i < m; ++i) hist[i0 + i] = (double)h[i];
+        });
         double nm = 0.0;
         for (int b = 0; b < c->nblk; ++b) {
             nm += host_block(c, b, chain)[qN];
@@ -2082,10 +2147,9 @@ int pimc_get_cartesian(pimc_ctx *c, int32_t chain, double *hist, int64_t *ndata)
     if (!c->d_cart) return set_err(c, PIMC_ERR_STATE, "Cartesian histogram not enabled");
     try {
         const long long nb = c->cart_per_chain;
-        std::vector<unsigned long long> h((size_t)nb);
-        HIPCHK(hipStreamSynchronize(c->stream));
-        HIPCHK(hipMemcpy(h.data(), c->d_cart + (size_t)chain * nb, sizeof(unsigned long long) * nb, hipMemcpyDeviceToHost));
-        for (long long i = 0; i < nb; ++i) hist[i] = (double)h[i];
+        from_device(c, c->d_cart + (size_t)chain * nb, (size_t)nb, [&](const unsigned long long *h, size_t i0, size_t m) {
+            for (size_t i = 0; i < m; ++i) hist[i0 + i] = (double)h[i];
+        });
         double nm = 0.0;
         for (int b = 0; b < c->nblk; ++b) {
             nm += host_block(c, b, chain)[qN];
@@ -2101,15 +2165,10 @@ int pimc_reset_estimators(pimc_ctx *c)
 {
     if (!c) return PIMC_ERR_ARG;
     try {
-        HIPCHK(hipStreamSynchronize(c->stream));
         c->nblk = 0;
         c->hblk_n = -1;
-        {
-            RunState rs{};
-            HIPCHK(hipMemcpy(&rs, c->d_rs, sizeof(RunState), hipMemcpyDeviceToHost));
-            rs.blk = 0;
-            h2d(c, c->d_rs, &rs, sizeof(RunState));
-        }
+        hipLaunchKernelGGL(k_reset_blocks, dim3(1), dim3(64), 0, c->stream, c->d_rs);
+        HIPCHK(hipGetLastError());
         // the histograms are cleared on the library stream, which the next run's kernels follow
         auto zero = [&](unsigned long long *p, long long n) {
             hipLaunchKernelGGL(k_zero_u64, dim3((unsigned)std::min<long long>(1024, (n + 255) / 256)), dim3(256), 0,
@@ -2118,7 +2177,6 @@ int pimc_reset_estimators(pimc_ctx *c)
         };
         if (c->d_radial) zero(c->d_radial, (long long)c->n_chains * c->opt.radial_bins);
         if (c->d_cart) zero(c->d_cart, (long long)c->n_chains * c->cart_per_chain);
-        HIPCHK(hipStreamSynchronize(c->stream));
     } catch (const HipError &e) {
         return hip_err(c, e);
     }
@@ -2150,37 +2208,40 @@ static int hook_move(pimc_ctx *c, int chain, int n, int j0, int m, const double 
     const int pot = h.pot, nseg = h.M / maxl;
     int sh = 0;
     while ((2 << sh) <= maxl) ++sh;
-    const size_t lds_fast = ((size_t)h.dim * tile_row_len(h.M, sh) + (size_t)nseg) * sizeof(float);
+    const size_t lds_fast = ((size_t)h.dim * tile_row_len(h.M, sh) + 2 * (size_t)nseg) * sizeof(float);
     try {
-        const int rows = com ? h.M : m + 1;
-        const size_t nout = (size_t)rows * h.dim + 5;
-        ensure_io(c, nout + (size_t)nin + 8);
-        double *d_in = c->d_io + nout;
-        HIPCHK(hipStreamSynchronize(c->stream));
-        h2d(c, d_in, in, sizeof(double) * nin);
+        const int rows = com ? h.M : m + 1, links = com ? h.M : m;
+        const size_t nrow = (size_t)rows * h.dim, nout = nrow + 6;
+        double *const pin = pinned<double>(c, (nout + (size_t)nin) * sizeof(double));
+        std::memcpy(pin + nout, in, sizeof(double) * nin);
+        size_t lds = hook_scratch(rows, links, h.dim, (int)tsize(c));
         HookArgs h = hook_args(c, chain);
+        if (!fast && lds > kHookLds) {
+            grow_device(c->d_work, c->work_elems, (lds + 7) / 8);
+            h.work = c->d_work;
+            lds = 0;
+        }
         h.n = n;
         h.j0 = j0;
         h.m = m;
         h.op = op;
-        h.in = d_in;
+        h.want_rows = r_out ? 1 : 0;
+        h.in = pin + nout;
         h.u = u;
-        h.out = c->d_io;
+        h.out = pin;
         if (fast) {
             h.m = com ? 0 : m;
             launch_tile_fast(c, h, maxl, pot, lds_fast);
         } else if (com) {
-            HOOK_DISPATCH(k_hook_com, dim3(1), dim3(64), 0, h);
+            HOOK_DISPATCH(k_hook_com, dim3(1), dim3(kHookThreads), lds, h);
         } else {
-            HOOK_DISPATCH(k_hook_reshape, dim3(1), dim3(64), 0, h);
+            HOOK_DISPATCH(k_hook_reshape, dim3(1), dim3(kHookThreads), lds, h);
         }
         HIPCHK(hipStreamSynchronize(c->stream));
-        std::vector<double> o(nout);
-        HIPCHK(hipMemcpy(o.data(), c->d_io, sizeof(double) * nout, hipMemcpyDeviceToHost));
-        if (r_out) std::memcpy(r_out, o.data(), sizeof(double) * (size_t)rows * c->dim);
-        if (w_out) std::memcpy(w_out, o.data() + (size_t)rows * c->dim, sizeof(double) * 4);
-        if (accepted) *accepted = o[(size_t)rows * c->dim + 4] != 0.0;
-        return check_status(c);
+        if (r_out) std::memcpy(r_out, pin, sizeof(double) * nrow);
+        if (w_out) std::memcpy(w_out, pin + nrow, sizeof(double) * 4);
+        if (accepted) *accepted = pin[nrow + 4] != 0.0;
+        return pin[nrow + 5] < 0.0 ? PIMC_OK : status_error(c, (int)pin[nrow + 5]);
     } catch (const HipError &e) {
         return hip_err(c, e);
     }
@@ -2220,15 +2281,14 @@ int pimc_interaction(pimc_ctx *c, int32_t chain, int32_t n, int32_t j, double *w
     if (n < 0 || n >= hc.N || j < 0 || j >= hc.M) return set_err(c, PIMC_ERR_ARG, "bad particle or slice");
     if ((rc = check_table(c, chain))) return rc;
     try {
-        ensure_io(c, 8);
-        HIPCHK(hipStreamSynchronize(c->stream));
+        double *const pin = pinned<double>(c, sizeof(double));
         HookArgs h = hook_args(c, chain);
         h.n = n;
         h.j0 = j;
-        h.out = c->d_io;
+        h.out = pin;
         HOOK_DISPATCH(k_hook_interaction, dim3(1), dim3(64), 0, h);
         HIPCHK(hipStreamSynchronize(c->stream));
-        HIPCHK(hipMemcpy(w, c->d_io, sizeof(double), hipMemcpyDeviceToHost));
+        *w = pin[0];
     } catch (const HipError &e) {
         return hip_err(c, e);
     }
@@ -2240,13 +2300,16 @@ int pimc_energy(pimc_ctx *c, int32_t chain, double *out)
     int rc = check_chain(c, chain);
     if (rc) return rc;
     try {
-        ensure_io(c, 8);
-        HIPCHK(hipStreamSynchronize(c->stream));
+        double *const pin = pinned<double>(c, 4 * sizeof(double));
         HookArgs h = hook_args(c, chain);
-        h.out = c->d_io;
-        HOOK_DISPATCH(k_hook_energy, dim3(1), dim3(256), 256 * sizeof(double), h);
+        const int nblk = hook_blocks(c, chain, c->ch[chain].pair == kPairGaussian ? 8 : 1);
+        h.part = c->d_hpart;
+        HOOK_DISPATCH(k_hook_energy, dim3(nblk), dim3(256), 0, h);
+        h.out = pin;
+        hipLaunchKernelGGL(k_hook_energy_fold, dim3(1), dim3(256), 0, c->stream, h, nblk);
+        HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(c->stream));
-        HIPCHK(hipMemcpy(out, c->d_io, sizeof(double) * 4, hipMemcpyDeviceToHost));
+        std::memcpy(out, pin, sizeof(double) * 4);
     } catch (const HipError &e) {
         return hip_err(c, e);
     }
@@ -2262,7 +2325,10 @@ int pimc_density(pimc_ctx *c, int32_t chain, int32_t nbins, double *dens, int64_
     const size_t nh = hc.dim == 1 ? (size_t)nbins : (size_t)nbins * nbins;
     unsigned long long *d_h = nullptr;
     try {
-        d_h = dalloc<unsigned long long>(nh);
+        // the context keeps the counts of histograms up to kScratchBins bins
+        const bool kept = nh <= (size_t)kScratchBins;
+        if (kept && !c->d_dens) c->d_dens = dalloc<unsigned long long>((size_t)kScratchBins);
+        d_h = kept ? c->d_dens : dalloc<unsigned long long>(nh);
         // cleared on the library stream, ahead of the counting kernel: a plain hipMemset runs on the
         // null stream, which the library's non-blocking stream does not wait for
         const unsigned fb = (unsigned)std::min<size_t>(1024, (nh + 255) / 256);
@@ -2281,15 +2347,14 @@ int pimc_density(pimc_ctx *c, int32_t chain, int32_t nbins, double *dens, int64_
         }
 #undef DENS
         HIPCHK(hipGetLastError());
-        HIPCHK(hipStreamSynchronize(c->stream));
-        std::vector<unsigned long long> hh(nh);
-        HIPCHK(hipMemcpy(hh.data(), d_h, sizeof(unsigned long long) * nh, hipMemcpyDeviceToHost));
-        dfree(d_h);
+        from_device(c, (const unsigned long long *)d_h, nh, [&](const unsigned long long *p, size_t i0, size_t m) {
+            for (size_t i = 0; i < m; ++i) dens[i0 + i] += (double)p[i];
+        });
+        if (!kept) dfree(d_h);
         d_h = nullptr;
-        for (size_t i = 0; i < nh; ++i) dens[i] += (double)hh[i];
         if (ndata) *ndata += hc.M;
     } catch (const HipError &e) {
-        dfree(d_h);
+        if (d_h != c->d_dens) dfree(d_h);
         return hip_err(c, e);
     }
     return PIMC_OK;
@@ -2349,20 +2414,29 @@ int pimc_adjoint(pimc_ctx *c, int32_t chain, double *dS_dr, double *dS_dparams, 
         return set_err(c, PIMC_ERR_ARG, "the adjoint is defined for a Gaussian pair action or none");
     const size_t nb = (size_t)hc.N * hc.dim * hc.M;
     try {
-        ensure_io(c, nb + 8);
-        HIPCHK(hipStreamSynchronize(c->stream));
+        ensure_io(c, nb + 3);
         HookArgs h = hook_args(c, chain);
+        const int lanes = hc.pair != kPairNone && c->prec == PIMC_FP64 ? hook_lanes<double>() : 1;
+        const int nblk = hook_blocks(c, chain, lanes);
+        h.part = c->d_hpart;
         h.out = c->d_io;
-        HOOK_DISPATCH(k_hook_adjoint, dim3(1), dim3(256), 256 * sizeof(double), h);
-        HIPCHK(hipStreamSynchronize(c->stream));
-        std::vector<double> o(nb + 3);
-        HIPCHK(hipMemcpy(o.data(), c->d_io, sizeof(double) * (nb + 3), hipMemcpyDeviceToHost));
-        if (dS_dr) std::memcpy(dS_dr, o.data(), sizeof(double) * nb);
+        HOOK_DISPATCH(k_hook_adjoint, dim3(nblk), dim3(256), 0, h);
+        h.out = c->d_io + nb;
+        hipLaunchKernelGGL(k_hook_adjoint_fold, dim3(1), dim3(256), 0, c->stream, h, nblk);
+        HIPCHK(hipGetLastError());
+        // without the gradient only the three sums after it come back
+        const size_t first = dS_dr ? 0 : nb;
+        double sums[3];
+        from_device(c, (const double *)c->d_io + first, nb + 3 - first, [&](const double *p, size_t i0, size_t m) {
+            const size_t at = first + i0, grad = at < nb ? std::min(m, nb - at) : 0;
+            if (grad > 0) std::memcpy(dS_dr + at, p, sizeof(double) * grad);
+            for (size_t i = grad; i < m; ++i) sums[at + i - nb] = p[i];
+        });
         if (dS_dparams) {
-            dS_dparams[0] = o[nb + 1];
-            dS_dparams[1] = o[nb + 2];
+            dS_dparams[0] = sums[1];
+            dS_dparams[1] = sums[2];
         }
-        if (S_out) *S_out = o[nb];
+        if (S_out) *S_out = sums[0];
     } catch (const HipError &e) {
         return hip_err(c, e);
     }

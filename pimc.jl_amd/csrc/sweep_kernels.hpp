@@ -64,6 +64,12 @@ __global__ void k_advance(RunState *rs, int nsweeps, int measure)
     }
 }
 
+// The next measured launch writes block 0 again (pimc_reset_estimators).
+__global__ void k_reset_blocks(RunState *rs)
+{
+    if (threadIdx.x == 0 && blockIdx.x == 0) rs->blk = 0;
+}
+
 struct TileDev {
     long long pos_off; // element offset of the tile's first particle
     int q0, np, M, nseg;
