@@ -1141,6 +1141,7 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
         HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         HIPCHK(hipEventCreate(&c->ev0));
         HIPCHK(hipEventCreate(&c->ev1));
+        (void)pinned<unsigned char>(c, 1);
         int cu = 256;
         {
             hipDeviceProp_t p;
@@ -2467,33 +2468,37 @@ int pimc_prop_int_terms(int32_t n, double r0, double r1, double g0, double tau, 
         ca[q] = cq / (1.0 + d * d);
         cb[q] = cq * d / (1.0 + d * d);
     }
-    double *dk = nullptr, *dca = nullptr, *dcb = nullptr, *dJ = nullptr, *dY = nullptr, *dout = nullptr;
+    // one allocation for the call: nodes and weights, the Bessel tables, the partial products, the table
+    double *d = nullptr;
     int rc = PIMC_OK;
     try {
-        dk = dalloc<double>(nk);
-        dca = dalloc<double>(nk);
-        dcb = dalloc<double>(nk);
-        dJ = dalloc<double>((size_t)n * nk);
-        dY = dalloc<double>((size_t)n * nk);
-        dout = dalloc<double>((size_t)n * n);
-        HIPCHK(hipMemcpy(dk, k.data(), sizeof(double) * nk, hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(dca, ca.data(), sizeof(double) * nk, hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(dcb, cb.data(), sizeof(double) * nk, hipMemcpyHostToDevice));
+        int dev = 0, cus = 256;
+        HIPCHK(hipGetDevice(&dev));
+        HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        const int tiles = prop_tiles(n), splits = prop_splits(n, nk, cus);
+        const size_t nb = (size_t)n * nk, npart = (size_t)splits * tiles * kPropTile * kPropTile;
+        d = dalloc<double>(3 * (size_t)nk + 2 * nb + npart + (size_t)n * n);
+        double *const dJ = d + 3 * (size_t)nk, *const dY = dJ + nb, *const dpart = dY + nb, *const dout = dpart + npart;
+        k.insert(k.end(), ca.begin(), ca.end());
+        k.insert(k.end(), cb.begin(), cb.end());
+        HIPCHK(hipMemcpy(d, k.data(), sizeof(double) * k.size(), hipMemcpyHostToDevice));
         const double h = (r1 - r0) / (n - 1);
         const long long tot = (long long)n * nk;
-        hipLaunchKernelGGL(k_prop_bessel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, nullptr, dk, nk, r0, h, n,
+        hipLaunchKernelGGL(k_prop_bessel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, nullptr, d, nk, r0, h, n,
                            dJ, dY);
         HIPCHK(hipGetLastError());
-        const unsigned nt = (unsigned)((n + kPropTile - 1) / kPropTile);
-        hipLaunchKernelGGL(k_prop_terms, dim3(nt, nt), dim3(kPropThreads), 0, nullptr, dJ, dY, dca, dcb, nk, n, dout);
+        hipLaunchKernelGGL(k_prop_terms, dim3((unsigned)tiles, (unsigned)splits), dim3(kPropThreads), 0, nullptr, dJ, dY,
+                           d + nk, d + 2 * (size_t)nk, nk, n, dpart);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipDeviceSynchronize());
+        hipLaunchKernelGGL(k_prop_fold, dim3((unsigned)tiles, kPropTile / 4), dim3(kPropThreads), 0, nullptr, dpart, splits,
+                           n, dout);
+        HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpy(terms, dout, sizeof(double) * n * n, hipMemcpyDeviceToHost));
     } catch (const HipError &e) {
         g_err = std::string(e.what) + ": " + hipGetErrorString(e.e);
         rc = PIMC_ERR_HIP;
     }
-    for (double *p : {dk, dca, dcb, dJ, dY, dout}) dfree(p);
+    dfree(d);
     return rc;
 }
 
