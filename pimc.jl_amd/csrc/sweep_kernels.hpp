@@ -16,6 +16,9 @@
 //    chain in HBM; particles are updated one after another, the segments (and
 //    links) of the current particle in parallel, pair sums through per-slice
 //    cell lists; swap tries follow the centre-of-mass pass.
+//  * k_sweep_ideal (ideal_kernels.hpp) takes the chains of k_sweep_whole that have
+//    no pair action (swap moves, whole-chain products) and fit in LDS, all
+//    particles at once.
 //  * the window kernels (window_kernels.hpp) take the Gaussian-pair chains with
 //    cell lists instead, many particles at once.
 #pragma once
@@ -1279,11 +1282,12 @@ struct ChainMeas {
     double link, V, rg, su, rgp, r2w;
 };
 
+// This thread's share of the sums over the beads [b0, b1) (all beads: b1 < 0) of a chain.
 template <typename T, int DIM, bool CELLS, typename PathT>
-__device__ inline ChainMeas measure_chain(const PathT &path, const Cells &C, const ChainDev &ch, const Prm<T> &P,
-                                          double *wbuf, unsigned long long *radial, int radial_bins,
-                                          double radial_winv, unsigned long long *cart, int cart_bins, int c,
-                                          int G = 1, const int *nxt = nullptr, int b0 = 0, int b1 = -1)
+__device__ inline ChainMeas measure_beads(const PathT &path, const Cells &C, const ChainDev &ch, const Prm<T> &P,
+                                          unsigned long long *radial, int radial_bins, double radial_winv,
+                                          unsigned long long *cart, int cart_bins, int c, int G, const int *nxt, int b0,
+                                          int b1)
 {
     const int N = ch.N, M = ch.M;
     if (b1 < 0) b1 = N * M;
@@ -1335,13 +1339,24 @@ __device__ inline ChainMeas measure_chain(const PathT &path, const Cells &C, con
             if (ok) atomicAdd(&cart[(size_t)c * stride + idx], 1ull);
         }
     }
+    return ChainMeas{l, v, g, su, rgp, r2w};
+}
+
+template <typename T, int DIM, bool CELLS, typename PathT>
+__device__ inline ChainMeas measure_chain(const PathT &path, const Cells &C, const ChainDev &ch, const Prm<T> &P,
+                                          double *wbuf, unsigned long long *radial, int radial_bins,
+                                          double radial_winv, unsigned long long *cart, int cart_bins, int c,
+                                          int G = 1, const int *nxt = nullptr, int b0 = 0, int b1 = -1)
+{
+    const ChainMeas t = measure_beads<T, DIM, CELLS>(path, C, ch, P, radial, radial_bins, radial_winv, cart, cart_bins, c,
+                                                     G, nxt, b0, b1);
     ChainMeas r;
-    r.link = block_sum(l, wbuf);
-    r.V = block_sum(v, wbuf);
-    r.rg = block_sum(g, wbuf);
-    r.su = block_sum(su, wbuf);
-    r.rgp = block_sum(rgp, wbuf);
-    r.r2w = block_sum(r2w, wbuf);
+    r.link = block_sum(t.link, wbuf);
+    r.V = block_sum(t.V, wbuf);
+    r.rg = block_sum(t.rg, wbuf);
+    r.su = block_sum(t.su, wbuf);
+    r.rgp = block_sum(t.rgp, wbuf);
+    r.r2w = block_sum(t.r2w, wbuf);
     return r;
 }
 
