@@ -42,6 +42,7 @@ struct ChainDev {
     int tab_n;
     int nbeam;
     int every_st, every_com, every_sw; // passes run on the sweeps s with s % every == 0
+    long long pair_off; // window chains: first pair slot (pair_row(N) of them) of the centre-of-mass pass
 };
 
 // Whether a pass with move weight 1/every runs in sweep sw (every >= 1).
@@ -110,6 +111,10 @@ template <typename T> struct Prm {
 
 __device__ __forceinline__ double fl(double x) { return floor(x); }
 __device__ __forceinline__ float fl(float x) { return floorf(x); }
+__device__ __forceinline__ double min_(double x, double y) { return __builtin_fmin(x, y); }
+__device__ __forceinline__ float min_(float x, float y) { return __builtin_fminf(x, y); }
+__device__ __forceinline__ double fma_(double x, double y, double z) { return __builtin_fma(x, y, z); }
+__device__ __forceinline__ float fma_(float x, float y, float z) { return __builtin_fmaf(x, y, z); }
 __device__ __forceinline__ double cpi(double x) { return cospi(x); }
 __device__ __forceinline__ float cpi(float x) { return cospif(x); }
 __device__ __forceinline__ double spi(double x) { return sinpi(x); }

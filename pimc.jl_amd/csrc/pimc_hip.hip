@@ -116,14 +116,20 @@ struct pimc_ctx {
     int *d_win_all = nullptr;
     int win_seg = 0, win_maxN = 0, win_maxM = 0, win_maxell = 0, win_maxM0 = 0;
     int cap_stage = 0, cap_cspec = 0, cap_cdec = 0;   // pair-slot pools of the three kernels
-    size_t lds_stage = 0, lds_cspec = 0, lds_cdec = 0, lds_cells = 0;
+    int rows_cspec = 64, nt_cspec = 512;              // k_com_spec: particles per block, threads
+    size_t lds_stage = 0, lds_cspec = 0, lds_cdec = 0, lds_cells = 0, lds_cbnd = 0;
     int cells_wpg = 4, win_ncell = 0;                 // k_cells_win: waves per workgroup, largest cell count
-    double *d_spec = nullptr;                         // centre of mass: Delta V + sum A per (particle, window)
-    void *d_wbnd = nullptr;                           // window bounds (float4) per (particle, window)
+    // centre-of-mass pass of the window chains (ComBuf)
+    double *d_spec = nullptr;                         // Delta V + sum A per (particle, window)
+    void *d_wbnd = nullptr, *d_rbnd = nullptr;        // bounds (float4) per (particle, window) and per particle
     int spec_nwin = 1;
-    unsigned char *d_cacc = nullptr;                  // centre of mass: accepted flag per particle
+    unsigned char *d_cacc = nullptr;                  // accepted flag per particle
     void *d_cshift = nullptr;                         // and its shift (2 per particle, arithmetic type)
-    void *d_pm = nullptr;                             // particle-major copy of the window chains' paths
+    int *d_ccnt = nullptr;                            // listed partners per particle
+    unsigned short *d_partner = nullptr;              // ... and the partners, per pair slot
+    void *d_cval = nullptr;                           // C per window and pair slot
+    // batches of a window group whose pair slots are in use together: win_all[first .. first + n)
+    std::vector<std::pair<int, int>> wg_batch[2];
     double *d_win_part = nullptr;                     // estimator partials of the window chains [chain][window][6]
     size_t lds_meas = 0;
     // The window chains in one group, or in two of about equal beads when there are two or more
@@ -606,6 +612,10 @@ void launch_meas(pimc_ctx *c, int sweep_off)
     }
 }
 
+// Pair slots of a window group's centre-of-mass pass held at a time (all windows of all pairs of a
+// batch of chains: 256 chains of N = 256, M = 128 in FP32 take 0.5 GiB).
+constexpr size_t kPairBytes = (size_t)4 << 30;
+
 // The stream of window group g.
 hipStream_t win_stream(const pimc_ctx *c, int g) { return g == 0 ? c->stream : c->stream2; }
 
@@ -668,15 +678,31 @@ template <typename T, int DIM> void launch_win_d(pimc_ctx *c, const SweepArgs &b
     hipLaunchKernelGGL((k_stage_win<T, DIM>), dim3((unsigned)c->win_seg, (unsigned)n), dim3(512), c->lds_stage, st,
                        w, c->cap_stage);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL((k_com_spec<T, DIM>), dim3((unsigned)c->spec_nwin, (unsigned)n), dim3(512), c->lds_cspec, st,
-                       w, c->d_spec, static_cast<float4 *>(c->d_wbnd), c->spec_nwin, c->cap_cspec,
-                       static_cast<T *>(c->d_pm));
-    HIPCHK(hipGetLastError());
-    if (stagger && g == 0) HIPCHK(hipEventRecord(stagger, st));
-    hipLaunchKernelGGL((k_com_dec<T, DIM>), dim3((unsigned)n), dim3(1024), c->lds_cdec, st, w,
-                       (const double *)c->d_spec, static_cast<const float4 *>(c->d_wbnd), c->spec_nwin, c->cap_cdec,
-                       kChunk, c->d_cacc, static_cast<T *>(c->d_cshift), static_cast<const T *>(c->d_pm));
-    HIPCHK(hipGetLastError());
+    ComBuf<T> B{};
+    B.wbnd = static_cast<float4 *>(c->d_wbnd);
+    B.rbnd = static_cast<float4 *>(c->d_rbnd);
+    B.shift = static_cast<T *>(c->d_cshift);
+    B.spec = c->d_spec;
+    B.cnt = c->d_ccnt;
+    B.partner = c->d_partner;
+    B.cval = static_cast<T *>(c->d_cval);
+    B.nwin = c->spec_nwin;
+    const unsigned blk = (unsigned)((c->win_maxN + 63) / 64);
+    for (const auto &[first, nb] : c->wg_batch[g]) {
+        SweepArgs v = w;
+        v.whole = c->d_win_all + first;
+        hipLaunchKernelGGL((k_com_bounds<T, DIM>), dim3(blk, (unsigned)nb), dim3(256), c->lds_cbnd, st, v, B);
+        HIPCHK(hipGetLastError());
+        hipLaunchKernelGGL((k_com_pairs<T, DIM>), dim3(blk, (unsigned)nb), dim3(256), 0, st, v, B);
+        HIPCHK(hipGetLastError());
+        hipLaunchKernelGGL((k_com_spec<T, DIM>), dim3((unsigned)c->spec_nwin, (unsigned)nb), dim3(c->nt_cspec),
+                           c->lds_cspec, st, v, B, c->rows_cspec, c->cap_cspec);
+        HIPCHK(hipGetLastError());
+        if (stagger && g == 0 && first + nb == c->wg_off[0] + n) HIPCHK(hipEventRecord(stagger, st));
+        hipLaunchKernelGGL((k_com_dec<T, DIM>), dim3((unsigned)nb), dim3(1024), c->lds_cdec, st, v, B, c->cap_cdec,
+                           c->d_cacc);
+        HIPCHK(hipGetLastError());
+    }
     const long long beads = (long long)c->win_maxM * c->win_maxN;
     hipLaunchKernelGGL((k_com_apply<T, DIM>), dim3((unsigned)((beads + 255) / 256), (unsigned)n), dim3(256), 0, st, w,
                        (const unsigned char *)c->d_cacc, static_cast<const T *>(c->d_cshift));
@@ -1276,8 +1302,8 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
                     const int N = std::max(c->win_maxN, h.N), ell = std::max(c->win_maxell, h.ell);
                     const int lc = std::max(com_win_len(std::max(c->win_maxM, h.M)), 8);
                     win = stage_lds(N, ell, h.dim, tsz, N).ck.end <= 160 * 1024 &&
-                          com_spec_lds(N, lc, h.dim, tsz, N).ck.end <= 160 * 1024 &&
-                          com_dec_lds(N, h.dim, tsz, N).ck.end <= 160 * 1024;
+                          com_spec_lds(N, lc, h.dim, tsz, 64, N).end <= 160 * 1024 &&
+                          com_dec_lds(N, tsz, N).end <= 160 * 1024;
                 }
                 if (cells) {
                     h.ncell = (int)ncell;
@@ -1477,14 +1503,21 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
                 return std::max(cap, N);
             };
             c->cap_stage = grow([&](int k) { return stage_lds(N, c->win_maxell, d, ts_, k).ck.end; }, 64 * 1024);
-            c->cap_cspec = grow([&](int k) { return com_spec_lds(N, lc, d, ts_, k).ck.end; }, 48 * 1024);
-            c->cap_cdec = grow([&](int k) { return com_dec_lds(N, d, ts_, k).ck.end; }, 128 * 1024);
+            // blocks of up to 256 particles, fewer where the masks do not leave room for the pool
+            c->rows_cspec = 256;
+            while (c->rows_cspec > 64 && com_spec_lds(N, lc, d, ts_, c->rows_cspec, N).end > 120 * 1024) c->rows_cspec >>= 1;
+            c->cap_cspec = grow([&](int k) { return com_spec_lds(N, lc, d, ts_, c->rows_cspec, k).end; }, 80 * 1024);
+            if (c->cap_cspec < 4 * N) // more than half of the LDS anyway: one workgroup per CU
+                c->cap_cspec = grow([&](int k) { return com_spec_lds(N, lc, d, ts_, c->rows_cspec, k).end; }, 128 * 1024);
+            c->cap_cdec = grow([&](int k) { return com_dec_lds(N, ts_, k).end; }, 128 * 1024);
             c->cap_meas = grow([&](int k) { return meas_win_lds(N, lc, d, ts_, k).ck.end; }, 48 * 1024);
             c->lds_meas = meas_win_lds(N, lc, d, ts_, c->cap_meas).ck.end;
             c->d_win_part = dalloc<double>(c->win_all.size() * (size_t)c->spec_nwin * 6);
             c->lds_stage = stage_lds(N, c->win_maxell, d, ts_, c->cap_stage).ck.end;
-            c->lds_cspec = com_spec_lds(N, lc, d, ts_, c->cap_cspec).ck.end;
-            c->lds_cdec = com_dec_lds(N, d, ts_, c->cap_cdec).ck.end;
+            c->lds_cspec = com_spec_lds(N, lc, d, ts_, c->rows_cspec, c->cap_cspec).end;
+            c->nt_cspec = c->lds_cspec > 80 * 1024 ? 1024 : 512;
+            c->lds_cdec = com_dec_lds(N, ts_, c->cap_cdec).end;
+            c->lds_cbnd = (size_t)c->spec_nwin * kBndPart * sizeof(float4);
             c->cells_wpg = 4;
             while (c->cells_wpg > 1 && (size_t)c->cells_wpg * c->win_ncell * 4 > 64 * 1024) c->cells_wpg >>= 1;
             c->lds_cells = (size_t)c->cells_wpg * std::max(c->win_ncell, 1) * 4;
@@ -1492,7 +1525,8 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
             HIPCHK(hipMalloc(&c->d_wbnd, (size_t)c->n_part * c->spec_nwin * sizeof(float4)));
             c->d_cacc = dalloc<unsigned char>((size_t)c->n_part);
             HIPCHK(hipMalloc(&c->d_cshift, (size_t)c->n_part * 2 * ts));
-            HIPCHK(hipMalloc(&c->d_pm, std::max<size_t>(1, (size_t)c->n_pos * ts)));
+            HIPCHK(hipMalloc(&c->d_rbnd, (size_t)c->n_part * sizeof(float4)));
+            c->d_ccnt = dalloc<int>((size_t)c->n_part);
             win_attrs(c);
             // groups: the shortest prefix of win_all holding at least half of the beads, when the
             // window chains fill at most half of the CUs (one decision workgroup a chain: with
@@ -1518,6 +1552,31 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
             c->wg_n[0] = split;
             c->wg_off[1] = split;
             c->wg_n[1] = nwc - split;
+            // pair slots: room for every pair of a chain and window, for as many chains of a group at
+            // a time as kPairBytes holds (at least one)
+            size_t slots = 0;
+            for (int g = 0; g < c->n_wgroup; ++g) {
+                const size_t limit = kPairBytes / ((size_t)c->spec_nwin * ts);
+                size_t used = 0, most = 0;
+                int first = c->wg_off[g];
+                const int end = c->wg_off[g] + c->wg_n[g];
+                for (int i = first; i < end; ++i) {
+                    ChainDev &h = c->ch[c->win_all[i]];
+                    const size_t n = pair_row(h.N);
+                    if (i > first && used + n > limit) {
+                        c->wg_batch[g].push_back({first, i - first});
+                        first = i;
+                        used = 0;
+                    }
+                    h.pair_off = (long long)(slots + used);
+                    used += n;
+                    most = std::max(most, used);
+                }
+                if (end > first) c->wg_batch[g].push_back({first, end - first});
+                slots += most;
+            }
+            c->d_partner = dalloc<unsigned short>(slots);
+            HIPCHK(hipMalloc(&c->d_cval, std::max<size_t>(1, slots) * c->spec_nwin * ts));
             std::vector<char> has_cells(n_chains, 0);
             for (int id : c->win_ids[0]) has_cells[id] = 1;
             for (int g = 0; g < c->n_wgroup; ++g) {
@@ -1589,7 +1648,7 @@ int pimc_destroy(pimc_ctx *c)
                     c->d_step, c->d_cnt, c->d_chain_meas, c->d_blocks, c->d_radial, c->d_cart, c->d_whole,
                     c->d_whole_cells, c->d_whole_brute, c->d_is_whole, c->d_cell_cnt, c->d_bins, c->d_cell_mem,
                     c->d_status, c->d_work, c->d_io, c->d_whole_lds, c->d_next, c->d_meas_ids, c->d_meas_part,
-                    c->d_cells_all, c->d_spec, c->d_wbnd, c->d_win_all, c->d_cacc, c->d_cshift, c->d_pm, c->d_win_part,
+                    c->d_cells_all, c->d_spec, c->d_wbnd, c->d_win_all, c->d_cacc, c->d_cshift, c->d_rbnd, c->d_ccnt, c->d_partner, c->d_cval, c->d_win_part,
                     c->d_beams, c->d_wg_cells[0], c->d_wg_cells[1], c->d_hpart, c->d_dens, c->d_ideal};
     for (void *p : ptrs) dfree(p);
     for (double *p : c->d_tab) dfree(p);

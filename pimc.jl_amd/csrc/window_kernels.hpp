@@ -25,12 +25,14 @@
 // are decided.  Every sum runs in a fixed order (partners by index), so the
 // result does not depend on thread timing.
 //
-// Centre of mass.  k_com_spec computes, by windows of the ring, every try's
-// Delta V + sum_q A against the configuration at the start of the phase and
-// the window bounds of the old rings; k_com_dec (one workgroup per chain)
-// adds, for each try, the C terms of its accepted earlier partners, over the
-// windows where their bounds (old and shifted) come within the cut-off, and
-// decides in rounds as above; k_com_apply moves the accepted rings.
+// Centre of mass.  The sums A and C over the whole ring are taken window by
+// window before any decision, for every pair of particles that can meet:
+// k_com_bounds bounds each particle's beads per window and per ring,
+// k_com_pairs lists the pairs p > q whose ring bounds (old or shifted) come
+// within the cut-off, k_com_spec evaluates, per window, the listed pairs whose
+// window bounds do, each pair once for A(p, q), A(q, p) and C(p, q), and
+// k_com_dec (one workgroup per chain) only adds the windows' values and decides
+// in rounds as above; k_com_apply moves the accepted rings.
 //
 // The cell lists are not used by these kernels; k_cells_win rebuilds them
 // (members by particle index) where the estimators or other callers need them.
@@ -140,6 +142,41 @@ template <typename T, int DIM> struct SliceTerm {
         return in ? mult * (ctau * (e + next.e)) : T(0);
     }
 };
+
+// Sums and products that keep their roundings: pair_window's forms, whatever
+// code surrounds them.
+template <typename T> __device__ __forceinline__ T add_(T x, T y)
+{
+#pragma clang fp contract(off)
+    return x + y;
+}
+template <typename T> __device__ __forceinline__ T sub_(T x, T y)
+{
+#pragma clang fp contract(off)
+    return x - y;
+}
+template <bool MULT, typename T> __device__ __forceinline__ T link_term(T mult, T ctau, T e0, T e1)
+{
+#pragma clang fp contract(off)
+    const T s = ctau * (e0 + e1);
+    return MULT ? mult * s : s;
+}
+__device__ __forceinline__ bool is_neg_zero(float x) { return __float_as_uint(x) == 0x80000000u; }
+__device__ __forceinline__ bool is_neg_zero(double x) { return __double_as_longlong(x) == (long long)0x8000000000000000ull; }
+
+// dist2 with the minimum taken by one instruction instead of a compare and a select.
+template <typename T> __device__ __forceinline__ T mindist_min(T x1, T x2, const Prm<T> &p)
+{
+    const T dx = fabs(x1 - x2);
+    return min_(p.twoL - dx, dx);
+}
+template <typename T, int DIM> __device__ __forceinline__ T dist2_min(const T *x, const T *y, const Prm<T> &P)
+{
+    const T d0 = mindist_min(x[0], y[0], P);
+    if (DIM == 1) return d0 * d0;
+    const T d1 = mindist_min(x[DIM - 1], y[DIM - 1], P);
+    return fma_(d0, d0, d1 * d1);
+}
 
 // A(p, q) and, for q < p (back), C(p, q) over the links 0..m-1 of one window.
 // bead(t, who, ro, rn): old and new bead of particle p (who 0) or q (who 1) at
@@ -444,29 +481,29 @@ __device__ inline int chunk_slots(ChunkPtr<T> &X, int pa, int N, int cap, int kc
     return nf;
 }
 
-// Decisions of the chunk's tries pa .. pa + nf - 1 in index order (wave 0).
-// Slots X.off[l] .. X.nb[l] hold try l's earlier partners by index with their
-// C values; acc[q] holds the decisions of the tries before the chunk.  A try
-// waits for its earlier partners inside the chunk that have a term within the
-// cut-off (the others add exactly zero).  Each round decides every try whose
-// such partners are decided; a try's sum takes the partners before the chunk
-// in index order, then the partners inside the chunk as they are accepted
-// (by round, in index order within a round), a fixed order.  Returns the
-// acceptance mask.
-template <typename T, typename Unif>
-__device__ inline unsigned long long chunk_decide(const ChunkPtr<T> &X, int pa, int nf, const unsigned char *acc,
-                                                  Unif unif)
+// Decisions of the chunk's tries pa .. pa + nf - 1 in index order (one wave,
+// lane l decides try pa + l).  Slots o0 .. o1 of pq, pc hold the try's earlier
+// partners by index (hit flag in bit 15) with their C values, sp its sum against
+// the configuration at the start, u its uniform; acc[q] holds the decisions of
+// the tries before the chunk.  A try waits for its earlier partners inside the
+// chunk that have a term within the cut-off (the others add exactly zero).  Each
+// round decides every try whose such partners are decided; a try's sum takes the
+// partners before the chunk in index order, then the partners inside the chunk as
+// they are accepted (by round, in index order within a round), a fixed order.
+// Returns the acceptance mask.
+template <typename T>
+__device__ inline unsigned long long chunk_decide(const unsigned short *pq, const T *pc, int o0, int o1, double sp, T u,
+                                                  int pa, int nf, const unsigned char *acc)
 {
     const int l = threadIdx.x & 63;
     const bool in = l < nf;
-    const int o0 = in ? X.off[l] : 0, o1 = in ? X.nb[l] : 0;
     T tot = T(0);
     unsigned long long dep = 0ull, pm = 0ull; // in-chunk partners with a term within the cut-off, all
     int si = o1;                              // first in-chunk partner's slot
     for (int i = o0; i < o1; ++i) {
-        const int qq = X.pq[i], q = qq & 0x7fff;
+        const int qq = pq[i], q = qq & 0x7fff;
         if (q < pa) {
-            if (acc[q]) tot += X.pc[i];
+            if (acc[q]) tot += pc[i];
         } else {
             if (si == o1) si = i;
             pm |= 1ull << (q - pa);
@@ -474,8 +511,6 @@ __device__ inline unsigned long long chunk_decide(const ChunkPtr<T> &X, int pa, 
         }
     }
     unsigned long long decided = nf >= 64 ? 0ull : (~0ull << nf), am = 0ull;
-    const double sp = in ? X.spec[l] : 0.0;
-    const T u = in ? unif(pa + l) : T(0);
     while (decided != ~0ull) {
         const bool ready = in && !((decided >> l) & 1ull) && (dep & ~decided) == 0ull;
         bool ok = false;
@@ -491,7 +526,7 @@ __device__ inline unsigned long long chunk_decide(const ChunkPtr<T> &X, int pa, 
             while (b) {
                 const int k = __ffsll((long long)b) - 1;
                 b &= b - 1;
-                tot += X.pc[si + __popcll(pm & ((1ull << k) - 1ull))];
+                tot += pc[si + __popcll(pm & ((1ull << k) - 1ull))];
             }
         }
     }
@@ -700,8 +735,10 @@ template <typename T, int DIM> __global__ void __launch_bounds__(512) k_stage_wi
         }
         __syncthreads();
         if (wave == 0) {
-            const unsigned long long am = chunk_decide<T>(X, pa, nf, acc, [&](int p) { return su[p]; });
             const int l = tid;
+            const bool in = l < nf;
+            const unsigned long long am = chunk_decide<T>(X.pq, X.pc, in ? X.off[l] : 0, in ? X.nb[l] : 0, in ? X.spec[l] : 0.0,
+                                                          in ? su[pa + l] : T(0), pa, nf, acc);
             if (l < nf) acc[pa + l] = (unsigned char)((am >> l) & 1ull);
             lacc += __popcll(am);
         }
@@ -734,56 +771,278 @@ __device__ __forceinline__ void com_try(const SweepArgs &a, int c, uint32_t sw, 
     u = Uniform<T>::get(y.z);
 }
 
-struct ComSpecLds {
-    size_t ob, sd, bnd, dv;
-    GridLds gr;
-    ChunkLds ck;
+// Index of pair (p, q = 0) among the pairs p > q of a chain.
+__host__ __device__ __forceinline__ size_t pair_row(int p) { return (size_t)p * (size_t)(p - 1) / 2; }
+
+// Buffers of the centre-of-mass kernels.  Per particle (window chains only, by
+// part_base) wbnd[. * nwin + w] bounds its old beads in window w, rbnd its old
+// ring, shift/unif hold its try, cnt the listed partners; per pair slot
+// (ChainDev::pair_off + pair_row(p) + k, the k-th listed partner of p by index)
+// partner; per window and slot (at nwin times the chain's pair offset)
+// cval: C of the window, with +0 for "no term within the cut-off" (a value of
+// zero with one is stored as -0).
+template <typename T> struct ComBuf {
+    float4 *wbnd, *rbnd;
+    T *shift;
+    double *spec; // [particle * nwin + w]: the window's Delta V + sum_q A
+    int *cnt;
+    unsigned short *partner;
+    T *cval;
+    int nwin;
+    __device__ __forceinline__ unsigned short *row(const ChainDev &ch, int p) const
+    {
+        return partner + ch.pair_off + pair_row(p);
+    }
+    __device__ __forceinline__ T *vals(const ChainDev &ch, int w) const
+    {
+        return cval + (size_t)ch.pair_off * nwin + (size_t)w * pair_row(ch.N);
+    }
 };
-__host__ __device__ inline ComSpecLds com_spec_lds(int N, int lc, int dim, int tsize, int cap)
+
+// Whether the bounds of two particles come within reach in one of the four
+// pairings of old and shifted beads.
+template <typename T, int DIM>
+__device__ __forceinline__ bool com_near(float4 A, const T *da, float4 B, const T *db, float h, float twoL, float inv2L)
 {
-    ComSpecLds L;
-    size_t o = 0;
-    L.ob = o;
-    o = align16(o + (size_t)(lc + 1) * N * dim * tsize);
-    L.sd = o;
-    o = align16(o + (size_t)N * dim * tsize);
-    L.bnd = o;
-    o = align16(o + (size_t)N * 16);
-    L.dv = o;
-    o = align16(o + (size_t)N * tsize);
-    L.gr = grid_lds(o, N, dim);
-    L.ck = chunk_lds(L.gr.end, N, cap, tsize, 1);
-    return L;
+    float fa[2], fb[2];
+    fa[0] = (float)da[0];
+    fb[0] = (float)db[0];
+    fa[1] = DIM > 1 ? (float)da[DIM - 1] : 0.f;
+    fb[1] = DIM > 1 ? (float)db[DIM - 1] : 0.f;
+    return bnd_near4<DIM>(A, fa, B, fb, h, twoL, inv2L);
 }
 
-// Phase 1 of the centre-of-mass moves: one workgroup per (window, chain),
-// windows of com_win_len(M) slices from slice 0.  spec[part * nwin + w]: the
-// window's Delta V + sum_q A of the particle's try against the configuration
-// at the start of the phase; wbnd[part * nwin + w]: the bound of the
-// particle's old beads in the window.
-template <typename T, int DIM>
-__global__ void __launch_bounds__(512) k_com_spec(SweepArgs a, double *spec, float4 *wbnd, int nwin, int cap, T *pm)
+constexpr int kBndPart = 64; // particles per workgroup of k_com_bounds
+
+// The tries' shifts and the bounds of the old beads: grid (particle blocks,
+// chains), 256 threads, four windows of 64 particles at a time (the particles of
+// a slice are consecutive in memory).  A window's bound: the middle of the beads'
+// extent, and the largest distance from it; a ring's: the same of its windows'
+// bounds, unwrapped against window 0's.
+template <typename T, int DIM> __global__ void __launch_bounds__(256) k_com_bounds(SweepArgs a, ComBuf<T> B)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const int c = a.whole[blockIdx.y];
     const ChainDev ch = a.chains[c];
-    const int w = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
+    const int N = ch.N, M = ch.M, lc = com_win_len(M), nw = com_nwin(M);
+    const int l = threadIdx.x & 63, p = blockIdx.x * kBndPart + l;
+    if ((int)blockIdx.x * kBndPart >= N) return;
+    const uint32_t sw = a.rs->sweep + (uint32_t)a.sweep_off;
+    if (!pass_on(ch.every_com, sw)) return; // no centre-of-mass pass in this sweep
+    const Prm<T> P = reinterpret_cast<const Prm<T> *>(a.prm)[c];
+    float4 *s_b = reinterpret_cast<float4 *>(smem); // [window][64]
+    const T *const gpath = reinterpret_cast<const T *>(a.pos) + ch.pos_off;
+    const size_t part = (size_t)ch.part_base + p;
+    for (int w = threadIdx.x >> 6; w < nw; w += 4) {
+        if (p >= N) continue;
+        const int s0 = w * lc, m = min(lc, M - s0);
+        T r0[DIM];
+        float lo[DIM], hi[DIM];
+        auto offset = [&](int t, float *o) {
+            int j = s0 + t;
+            if (j >= M) j -= M;
+            const T *r = gpath + ((size_t)j * N + p) * DIM;
+#pragma unroll
+            for (int e = 0; e < DIM; ++e) o[e] = (float)signed_mindist(r[e], r0[e], P);
+        };
+#pragma unroll
+        for (int e = 0; e < DIM; ++e) {
+            r0[e] = gpath[((size_t)s0 * N + p) * DIM + e];
+            lo[e] = hi[e] = 0.f;
+        }
+        for (int t = 1; t <= m; ++t) {
+            float o[DIM];
+            offset(t, o);
+#pragma unroll
+            for (int e = 0; e < DIM; ++e) {
+                lo[e] = fminf(lo[e], o[e]);
+                hi[e] = fmaxf(hi[e], o[e]);
+            }
+        }
+        float r2 = 0.f;
+        for (int t = 0; t <= m; ++t) {
+            float o[DIM], d2 = 0.f;
+            offset(t, o);
+#pragma unroll
+            for (int e = 0; e < DIM; ++e) {
+                const float x = o[e] - 0.5f * (lo[e] + hi[e]);
+                d2 += x * x;
+            }
+            r2 = fmaxf(r2, d2);
+        }
+        const float4 b = make_float4((float)r0[0] + 0.5f * (lo[0] + hi[0]),
+                                     DIM > 1 ? (float)r0[DIM - 1] + 0.5f * (lo[DIM - 1] + hi[DIM - 1]) : 0.f,
+                                     sqrtf(r2) * 1.00001f, 0.f);
+        s_b[w * 64 + l] = b;
+        B.wbnd[part * B.nwin + w] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64 || p >= N) return;
+    const float twoL = (float)(2.0 * ch.L), inv2L = 1.0f / twoL;
+    const float4 b0 = s_b[l];
+    float lx = 0.f, hx = 0.f, ly = 0.f, hy = 0.f;
+    for (int w = 1; w < nw; ++w) {
+        const float4 b = s_b[w * 64 + l];
+        const float x = mi_f(b.x - b0.x, twoL, inv2L), y = DIM > 1 ? mi_f(b.y - b0.y, twoL, inv2L) : 0.f;
+        lx = fminf(lx, x), hx = fmaxf(hx, x);
+        ly = fminf(ly, y), hy = fmaxf(hy, y);
+    }
+    const float cx = 0.5f * (lx + hx), cy = 0.5f * (ly + hy);
+    float r = 0.f;
+    for (int w = 0; w < nw; ++w) {
+        const float4 b = s_b[w * 64 + l];
+        const float x = mi_f(b.x - b0.x, twoL, inv2L) - cx, y = (DIM > 1 ? mi_f(b.y - b0.y, twoL, inv2L) : 0.f) - cy;
+        r = fmaxf(r, sqrtf(x * x + y * y) + b.z);
+    }
+    B.rbnd[part] = make_float4(b0.x + cx, b0.y + cy, r * 1.00001f, 0.f);
+    T d[DIM], u;
+    com_try<T, DIM>(a, c, sw, p, d, u);
+#pragma unroll
+    for (int e = 0; e < DIM; ++e) B.shift[part * 2 + e] = d[e];
+}
+
+// The listed partners q < p of each particle, by index: grid (blocks of 64
+// particles, chains), 256 threads, one wave per particle and 64 partners at a time.
+template <typename T, int DIM> __global__ void __launch_bounds__(256) k_com_pairs(SweepArgs a, ComBuf<T> B)
+{
+    const int c = a.whole[blockIdx.y];
+    const ChainDev ch = a.chains[c];
+    const int N = ch.N, lane = threadIdx.x & 63;
+    if (!pass_on(ch.every_com, a.rs->sweep + (uint32_t)a.sweep_off)) return;
+    const float h = (float)ch.h, twoL = (float)(2.0 * ch.L), inv2L = 1.0f / twoL;
+    const float4 *rb = B.rbnd + ch.part_base;
+    const T *sd = B.shift + (size_t)ch.part_base * 2;
+    const int p1 = min(N, ((int)blockIdx.x + 1) * 64);
+    for (int p = (int)blockIdx.x * 64 + (threadIdx.x >> 6); p < p1; p += 4) {
+        unsigned short *row = B.row(ch, p);
+        const float4 A = rb[p];
+        const T da[2] = {sd[p * 2], DIM > 1 ? sd[p * 2 + 1] : T(0)};
+        int n = 0;
+        for (int q0 = 0; q0 < p; q0 += 64) {
+            const int q = q0 + lane;
+            const bool ok = q < p && com_near<T, DIM>(A, da, rb[q], sd + q * 2, h, twoL, inv2L);
+            const unsigned long long bal = __ballot(ok);
+            if (ok) row[n + __popcll(bal & ((1ull << lane) - 1ull))] = (unsigned short)q;
+            n += __popcll(bal);
+        }
+        if (lane == 0) B.cnt[ch.part_base + p] = n;
+    }
+}
+
+// LDS of k_com_spec for blocks of R particles (rows) and a pool of cap pairs:
+// beads of the window's slices, shifts, sums, masks of the rows' partners in
+// reach (words of 64 list entries) and of each particle's rows (words of 64
+// rows), then the pool: row, list index, partner and the two A values.
+struct ComSpecLds {
+    size_t ob, sd, sp, rmask, roff, cmask, coff, misc, prow, pk, pq, pa, pb, end;
+};
+__host__ __device__ inline ComSpecLds com_spec_lds(int N, int lc, int dim, int tsize, int R, int cap)
+{
+    ComSpecLds L;
+    size_t o = 0;
+    auto take = [&](size_t bytes) {
+        const size_t at = o;
+        o = align16(o + bytes);
+        return at;
+    };
+    const int nq = (N + 63) / 64;
+    L.ob = take((size_t)(lc + 1) * N * dim * tsize);
+    L.sd = take((size_t)N * dim * tsize);
+    L.sp = take((size_t)N * 8);
+    L.rmask = take((size_t)R * nq * 8);
+    L.roff = take((size_t)(R + 1) * 4);
+    L.cmask = take((size_t)N * (R / 64) * 8);
+    L.coff = take((size_t)N * 2);
+    L.misc = take(16);
+    L.prow = take((size_t)cap);
+    L.pk = take((size_t)cap * 2);
+    L.pq = take((size_t)cap * 2);
+    L.pa = take((size_t)cap * tsize);
+    L.pb = take((size_t)cap * tsize);
+    L.end = o;
+    return L;
+}
+
+// A(p, q), A(q, p) and C(p, q) of one pair over the links 0 .. m - 1 of a window:
+// pair_window's terms, the pairings of old (o) and new (n) beads each evaluated
+// once for both particles.  MULT: chains with nbins < 3, whose terms carry a
+// stencil multiplicity.
+template <typename T, int DIM, bool MULT, typename BeadFn>
+__device__ __forceinline__ void pair_window_both(BeadFn bead, int m, const Prm<T> &P, int nbins, T &Apq, T &Aqp, T &C,
+                                                 bool &hit)
+{
+    const T ctau = T(-0.5) * P.tau;
+    T e0[4], u0[4]; // the previous slice's pair potential and multiplicity: oo, no, on, nn
+    bool in0[4];
+    Apq = Aqp = C = T(0);
+    hit = false;
+    for (int t = 0; t <= m; ++t) {
+        T po[DIM], pn[DIM], qo[DIM], qn[DIM];
+        bead(t, 0, po, pn);
+        bead(t, 1, qo, qn);
+        const T *x[4] = {po, pn, po, pn}, *y[4] = {qo, qo, qn, qn};
+        T e[4], u[4], tl[4];
+        bool in[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const T d2 = dist2_min<T, DIM>(x[k], y[k], P);
+            in[k] = d2 <= P.h2;
+            e[k] = vpair_r2(d2, P);
+            u[k] = MULT ? stencil_mult<T, DIM>(x[k], y[k], P, nbins) : T(1);
+        }
+        if (t > 0) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) tl[k] = in0[k] ? link_term<MULT>(u0[k], ctau, e0[k], e[k]) : T(0);
+            const T a1 = sub_(tl[1], tl[0]);
+            Apq = add_(Apq, a1);
+            Aqp = add_(Aqp, sub_(tl[2], tl[0]));
+            C = add_(C, sub_(sub_(tl[3], tl[2]), a1));
+        }
+        if (t < m) hit = hit || in[0] || in[1] || in[2] || in[3];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            e0[k] = e[k];
+            in0[k] = in[k];
+            if (MULT) u0[k] = u[k];
+        }
+    }
+}
+
+// Phase 1 of the centre-of-mass moves: one workgroup per (window, chain),
+// windows of com_win_len(M) slices from slice 0, every try against the
+// configuration at the start of the phase.  Blocks of at most R particles whose
+// pairs in reach fit the pool; per block the pairs are found from the list by
+// window bounds, evaluated one per thread, and each particle's sum takes its
+// partners by index (the block's own rows first, then the rows that name it).
+// The pair terms are VALU work, four pairings of two beads a slice; a pool of the
+// whole window's pairs keeps the threads evenly loaded.
+template <typename T, int DIM>
+__global__ void __launch_bounds__(1024) k_com_spec(SweepArgs a, ComBuf<T> B, int R, int cap)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int c = a.whole[blockIdx.y];
+    const ChainDev ch = a.chains[c];
+    const int w = blockIdx.x, tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nwv = nt >> 6;
     const int M = ch.M, N = ch.N, lc = com_win_len(M);
     if (w * lc >= M) return;
     const int m = min(lc, M - w * lc), s0 = w * lc;
-    const uint32_t sw = a.rs->sweep + (uint32_t)a.sweep_off;
-    if (!pass_on(ch.every_com, sw)) return; // no centre-of-mass pass in this sweep
-    if (cap < N) {
+    if (!pass_on(ch.every_com, a.rs->sweep + (uint32_t)a.sweep_off)) return; // no centre-of-mass pass in this sweep
+    if (cap < N) { // the host sizes the pool for every particle's partners
         if (tid == 0) atomicOr(a.status + c, 2);
         return;
     }
     const Prm<T> P = reinterpret_cast<const Prm<T> *>(a.prm)[c];
-    const ComSpecLds L = com_spec_lds(N, lc, DIM, (int)sizeof(T), cap);
-    T *ob = reinterpret_cast<T *>(smem + L.ob);
-    T *sd = reinterpret_cast<T *>(smem + L.sd);
-    float4 *bnd = reinterpret_cast<float4 *>(smem + L.bnd);
-    T *dvs = reinterpret_cast<T *>(smem + L.dv);
-    ChunkPtr<T> X(smem, L.ck);
+    const ComSpecLds L = com_spec_lds(N, lc, DIM, (int)sizeof(T), R, cap);
+    T *const ob = reinterpret_cast<T *>(smem + L.ob), *const sd = reinterpret_cast<T *>(smem + L.sd);
+    double *const sp = reinterpret_cast<double *>(smem + L.sp);
+    unsigned long long *const rmask = reinterpret_cast<unsigned long long *>(smem + L.rmask);
+    unsigned long long *const cmask = reinterpret_cast<unsigned long long *>(smem + L.cmask);
+    int *const roff = reinterpret_cast<int *>(smem + L.roff), *const misc = reinterpret_cast<int *>(smem + L.misc);
+    unsigned short *const coff = reinterpret_cast<unsigned short *>(smem + L.coff);
+    unsigned char *const prow = smem + L.prow;
+    unsigned short *const pk = reinterpret_cast<unsigned short *>(smem + L.pk);
+    unsigned short *const pq = reinterpret_cast<unsigned short *>(smem + L.pq);
+    T *const pa_ = reinterpret_cast<T *>(smem + L.pa), *const pb_ = reinterpret_cast<T *>(smem + L.pb);
     const T *const gpath = reinterpret_cast<const T *>(a.pos) + ch.pos_off;
     for (int t = 0; t <= m; ++t) {
         const int j = (s0 + t) % M;
@@ -791,79 +1050,100 @@ __global__ void __launch_bounds__(512) k_com_spec(SweepArgs a, double *spec, flo
         T *dst = ob + (size_t)t * N * DIM;
         for (int i = tid; i < N * DIM; i += nt) dst[i] = src[i];
     }
-    __syncthreads();
-    // the window's slices particle-major for the decision kernel: a particle's
-    // consecutive beads share cache lines there
-    {
-        T *dst = pm + ch.pos_off;
-        for (int it = tid; it < N * m; it += nt) {
-            const int p = it / m, t = it - p * m;
+    const size_t part = (size_t)ch.part_base;
+    for (int p = tid; p < N; p += nt)
 #pragma unroll
-            for (int e = 0; e < DIM; ++e) dst[((size_t)p * M + s0 + t) * DIM + e] = ob[((size_t)t * N + p) * DIM + e];
-        }
-    }
+        for (int e = 0; e < DIM; ++e) sd[p * DIM + e] = B.shift[(part + p) * 2 + e];
+    __syncthreads();
     for (int p = tid; p < N; p += nt) {
-        T d[DIM], u;
-        com_try<T, DIM>(a, c, sw, p, d, u);
         T dv = T(0);
-        float mean[DIM] = {};
         for (int t = 0; t < m; ++t) {
             T ro[DIM], rn[DIM];
 #pragma unroll
             for (int e = 0; e < DIM; ++e) {
                 ro[e] = ob[((size_t)t * N + p) * DIM + e];
-                rn[e] = teleport(ro[e] + d[e], P);
+                rn[e] = teleport(ro[e] + sd[p * DIM + e], P);
             }
             dv += -P.tau * (potV<T, DIM>(rn, P) - potV<T, DIM>(ro, P));
         }
-        for (int t = 0; t <= m; ++t) {
-#pragma unroll
-            for (int e = 0; e < DIM; ++e)
-                mean[e] += (float)signed_mindist(ob[((size_t)t * N + p) * DIM + e], ob[(size_t)p * DIM + e], P);
-        }
-#pragma unroll
-        for (int e = 0; e < DIM; ++e) mean[e] /= (float)(m + 1);
-        float r2 = 0.f;
-        for (int t = 0; t <= m; ++t) {
-            float d2 = 0.f;
-#pragma unroll
-            for (int e = 0; e < DIM; ++e) {
-                const float o = (float)signed_mindist(ob[((size_t)t * N + p) * DIM + e], ob[(size_t)p * DIM + e], P) - mean[e];
-                d2 += o * o;
-            }
-            r2 = fmaxf(r2, d2);
-        }
-        const float4 b = make_float4((float)ob[(size_t)p * DIM] + mean[0],
-                                     DIM > 1 ? (float)ob[(size_t)p * DIM + DIM - 1] + mean[DIM - 1] : 0.f, sqrtf(r2), 0.f);
-        bnd[p] = b;
-        wbnd[((size_t)ch.part_base + p) * nwin + w] = b;
-#pragma unroll
-        for (int e = 0; e < DIM; ++e) sd[p * DIM + e] = d[e];
-        dvs[p] = dv;
+        sp[p] = (double)dv;
     }
-    __syncthreads();
     const float h = (float)ch.h, twoL = (float)(2.0 * ch.L), inv2L = 1.0f / twoL;
-    // grid of the bounds of old and shifted beads together (centre halfway, radius
-    // grown by half the shift): both of a try's pairings lie within them
-    WinGrid G(smem, L.gr);
-    grid_build<DIM>(G, N, h, twoL, inv2L, [&](int p, float &x, float &y, float &r) {
-        const float4 b = bnd[p];
-        const float dx = (float)sd[p * DIM], dy = DIM > 1 ? (float)sd[p * DIM + DIM - 1] : 0.f;
-        x = b.x + 0.5f * dx;
-        y = b.y + 0.5f * dy;
-        r = (b.z + 0.5f * sqrtf(dx * dx + dy * dy)) * 1.00001f;
-    });
+    const int nq = (N + 63) / 64, nc = R / 64; // words of a row mask, of a column mask
+    T *const cval = B.vals(ch, w);
     for (int pa = 0; pa < N;) {
-        const int nf = chunk_slots<DIM>(X, pa, N, cap, kChunk, [&](int p, int q) {
-            if (q == p) return false;
-            const float4 A = bnd[p], B = bnd[q];
-            const float dx = (float)sd[p * DIM], dy = DIM > 1 ? (float)sd[p * DIM + DIM - 1] : 0.f;
-            return bnd_near<DIM>(A.x, A.y, A.z, B.x, B.y, B.z, h, twoL, inv2L) ||
-                   bnd_near<DIM>(A.x + dx, A.y + dy, A.z, B.x, B.y, B.z, h, twoL, inv2L);
-        }, &G);
-        const int total = X.misc[1];
+        const int nr = min(R, N - pa);
+        for (int i = tid; i < N * nc; i += nt) cmask[i] = 0ull;
+        // partners in reach of each row; the others' C is zero
+        for (int l = wave; l < nr; l += nwv) {
+            const int p = pa + l, n = B.cnt[part + p];
+            const unsigned short *row = B.row(ch, p);
+            const float4 bp = B.wbnd[(part + p) * B.nwin + w];
+            int cnt = 0;
+            for (int k0 = 0; k0 < n; k0 += 64) {
+                const int k = k0 + lane;
+                bool ok = false;
+                if (k < n) {
+                    const int q = row[k];
+                    ok = com_near<T, DIM>(bp, sd + p * DIM, B.wbnd[(part + q) * B.nwin + w], sd + q * DIM, h, twoL, inv2L);
+                    if (!ok) cval[pair_row(p) + k] = T(0);
+                }
+                const unsigned long long bal = __ballot(ok);
+                if (lane == 0) rmask[(size_t)l * nq + (k0 >> 6)] = bal;
+                cnt += __popcll(bal);
+            }
+            if (lane == 0) roff[l + 1] = cnt;
+        }
+        __syncthreads();
+        if (wave == 0) { // prefix; the rows whose pairs fit
+            int base = 0, nf = 0;
+            for (int l0 = 0; l0 < nr; l0 += 64) {
+                const int l = l0 + lane, v = l < nr ? roff[l + 1] : 0;
+                int tot;
+                const int pre = wave_prefix(v, lane, tot);
+                if (l < nr) roff[l + 1] = base + pre + v;
+                nf += __popcll(__ballot(l < nr && base + pre + v <= cap));
+                base += tot;
+            }
+            if (lane == 0) {
+                roff[0] = 0;
+                misc[0] = nf;
+            }
+        }
+        __syncthreads();
+        const int nf = misc[0], total = roff[nf];
+        for (int l = wave; l < nf; l += nwv) {
+            const int p = pa + l, n = B.cnt[part + p];
+            const unsigned short *row = B.row(ch, p);
+            int at = roff[l];
+            for (int k0 = 0; k0 < n; k0 += 64) {
+                const unsigned long long bal = rmask[(size_t)l * nq + (k0 >> 6)];
+                if ((bal >> lane) & 1ull) {
+                    const int s = at + __popcll(bal & ((1ull << lane) - 1ull)), q = row[k0 + lane];
+                    prow[s] = (unsigned char)l;
+                    pk[s] = (unsigned short)(k0 + lane);
+                    pq[s] = (unsigned short)q;
+                    atomicOr(cmask + (size_t)q * nc + (l >> 6), 1ull << (l & 63));
+                }
+                at += __popcll(bal);
+            }
+        }
+        __syncthreads();
+        if (wave == 0) { // where each particle's rows start
+            int base = 0;
+            for (int q0 = 0; q0 < N; q0 += 64) {
+                const int q = q0 + lane;
+                int v = 0, tot;
+                if (q < N)
+                    for (int k = 0; k < nc; ++k) v += __popcll(cmask[(size_t)q * nc + k]);
+                const int pre = wave_prefix(v, lane, tot);
+                if (q < N) coff[q] = (unsigned short)(base + pre);
+                base += tot;
+            }
+        }
+        __syncthreads();
         for (int i = tid; i < total; i += nt) {
-            const int p = pa + X.po[i], q = X.pq[i];
+            const int l = prow[i], p = pa + l, q = pq[i];
             auto bead = [&](int t, int who, T *ro, T *rn) {
                 const int k = who ? q : p;
 #pragma unroll
@@ -872,32 +1152,43 @@ __global__ void __launch_bounds__(512) k_com_spec(SweepArgs a, double *spec, flo
                     rn[e] = teleport(ro[e] + sd[k * DIM + e], P);
                 }
             };
-            T A, C;
+            T Apq, Aqp, C;
             bool hit;
-            pair_window<T, DIM, 1>(bead, m, false, P, ch.nbins, A, C, hit);
-            X.pa[i] = A;
+            if (ch.nbins >= 3) pair_window_both<T, DIM, false>(bead, m, P, ch.nbins, Apq, Aqp, C, hit);
+            else pair_window_both<T, DIM, true>(bead, m, P, ch.nbins, Apq, Aqp, C, hit);
+            int at = coff[q];
+            for (int k = 0; k < (l >> 6); ++k) at += __popcll(cmask[(size_t)q * nc + k]);
+            at += __popcll(cmask[(size_t)q * nc + (l >> 6)] & ((1ull << (l & 63)) - 1ull));
+            pa_[i] = Apq;
+            pb_[at] = Aqp;
+            cval[pair_row(p) + pk[i]] = !hit ? T(0) : (C == T(0) ? T(-0.0) : C);
         }
         __syncthreads();
-        if (tid < nf) {
-            const int p = pa + tid, o0 = X.off[tid], o1 = o0 + X.cnt[tid];
-            double sp = (double)dvs[p];
-            for (int i = o0; i < o1; ++i) sp += (double)X.pa[i];
-            spec[((size_t)ch.part_base + p) * nwin + w] = sp;
+        for (int x = tid; x < N; x += nt) {
+            double s = sp[x];
+            if (x >= pa && x < pa + nf)
+                for (int i = roff[x - pa]; i < roff[x - pa + 1]; ++i) s += (double)pa_[i];
+            int n = 0;
+            for (int k = 0; k < nc; ++k) n += __popcll(cmask[(size_t)x * nc + k]);
+            for (int i = coff[x]; i < coff[x] + n; ++i) s += (double)pb_[i];
+            sp[x] = s;
         }
         __syncthreads();
         pa += nf;
     }
+    for (int p = tid; p < N; p += nt) B.spec[(part + p) * B.nwin + w] = sp[p];
 }
 
-// Items of the decision kernel: (slot, window) pairs whose bounds come within
-// reach, taken kItemBatch at a time.
-constexpr int kItemBatch = 2048;
-
+// LDS of k_com_dec: the tries' sums, uniforms and decisions, then two chunk
+// buffers of cap pairs each.
 struct ComDecLds {
-    size_t spec, su, sd, rb, acc, pwb, wm, ioff, hitf, cw, hw;
-    ChunkLds ck;
+    size_t spec, su, acc, off, ck[2], end;
 };
-__host__ __device__ inline ComDecLds com_dec_lds(int N, int dim, int tsize, int cap)
+__host__ __device__ inline size_t com_dec_chunk(int cap, int tsize)
+{
+    return align16((size_t)cap * tsize) + align16((size_t)cap * 2) + align16((kChunk + 1) * 4) + 16;
+}
+__host__ __device__ inline ComDecLds com_dec_lds(int N, int tsize, int cap)
 {
     ComDecLds L;
     size_t o = 0;
@@ -905,42 +1196,29 @@ __host__ __device__ inline ComDecLds com_dec_lds(int N, int dim, int tsize, int 
     o = align16(o + (size_t)N * 8);
     L.su = o;
     o = align16(o + (size_t)N * tsize);
-    L.sd = o;
-    o = align16(o + (size_t)N * dim * tsize);
-    L.rb = o;
-    o = align16(o + (size_t)N * 16);
     L.acc = o;
     o = align16(o + (size_t)N);
-    L.pwb = o; // window bounds of the chunk's particles, kChunk x 32
-    o = align16(o + (size_t)kChunk * 32 * 16);
-    L.wm = o; // per slot: mask of the windows to evaluate
-    o = align16(o + (size_t)cap * 4);
-    L.ioff = o; // per slot: first item
-    o = align16(o + (size_t)cap * 4);
-    L.hitf = o; // per slot: a term within the cut-off
-    o = align16(o + (size_t)cap);
-    L.cw = o; // per item of a batch: C of the window
-    o = align16(o + (size_t)kItemBatch * tsize);
-    L.hw = o;
-    o = align16(o + (size_t)kItemBatch);
-    L.ck = chunk_lds(o, N, cap, tsize, 1);
+    for (int k = 0; k < 2; ++k) {
+        L.ck[k] = o;
+        o += com_dec_chunk(cap, tsize);
+    }
+    L.end = o;
     return L;
 }
 
-// Phase 2 of the centre-of-mass moves: one workgroup per chain.  Per try, the
-// C terms of its accepted earlier partners whose ring bounds (old or shifted)
-// come within the cut-off, summed over the windows where their window bounds
-// do; the tries are decided in chunks of rounds.  cacc[part]: 1 when the
-// particle's try was accepted, cshift[part * 2 + e] its shift.
+// Phase 2 of the centre-of-mass moves: one workgroup per chain.  Per chunk of 64
+// tries the listed pairs' C values are added over the windows (window order; zero
+// outside reach) into LDS, and one wave decides the chunk in rounds while the
+// other waves fetch the next chunk's.  What bounds it is the serial chain of
+// rounds of that wave.  cacc[part]: 1 when the particle's try was accepted.
 template <typename T, int DIM>
-__global__ void __launch_bounds__(1024) k_com_dec(SweepArgs a, const double *spec, const float4 *wbnd, int nwin,
-                                                   int cap, int kc, unsigned char *cacc, T *cshift, const T *pm)
+__global__ void __launch_bounds__(1024) k_com_dec(SweepArgs a, ComBuf<T> B, int cap, unsigned char *cacc)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const int c = a.whole[blockIdx.x];
     const ChainDev ch = a.chains[c];
-    const int N = ch.N, M = ch.M, tid = threadIdx.x, nt = blockDim.x, wave = tid >> 6;
-    const int lc = com_win_len(M), nw = com_nwin(M);
+    const int N = ch.N, nw = com_nwin(ch.M), tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6;
+    const int nwv = nt >> 6;
     const uint32_t sw = a.rs->sweep + (uint32_t)a.sweep_off;
     if (!pass_on(ch.every_com, sw)) return; // no centre-of-mass pass in this sweep: no tries
     if (cap < N) {
@@ -948,191 +1226,89 @@ __global__ void __launch_bounds__(1024) k_com_dec(SweepArgs a, const double *spe
         return;
     }
     const Prm<T> P = reinterpret_cast<const Prm<T> *>(a.prm)[c];
-    const ComDecLds L = com_dec_lds(N, DIM, (int)sizeof(T), cap);
-    double *s_spec = reinterpret_cast<double *>(smem + L.spec);
-    T *su = reinterpret_cast<T *>(smem + L.su);
-    T *sd = reinterpret_cast<T *>(smem + L.sd);
-    float4 *rb = reinterpret_cast<float4 *>(smem + L.rb);
-    unsigned char *acc = smem + L.acc;
-    float4 *pwb = reinterpret_cast<float4 *>(smem + L.pwb);
-    unsigned *s_wm = reinterpret_cast<unsigned *>(smem + L.wm);
-    int *s_ioff = reinterpret_cast<int *>(smem + L.ioff);
-    unsigned char *s_hitf = smem + L.hitf;
-    T *s_cw = reinterpret_cast<T *>(smem + L.cw);
-    unsigned char *s_hw = smem + L.hw;
-    ChunkPtr<T> X(smem, L.ck);
-    const T *ring = pm + ch.pos_off; // particle-major copy of the path: [particle][slice][d]
-    const float h = (float)ch.h, twoL = (float)(2.0 * ch.L), inv2L = 1.0f / twoL;
-    const float4 *wb = wbnd + (size_t)ch.part_base * nwin;
-    // per try: phase 1's value (windows in order), shift and uniform, and the ring bound
-    // from the window bounds (centres unwrapped against window 0's)
+    const ComDecLds L = com_dec_lds(N, (int)sizeof(T), cap);
+    double *const s_spec = reinterpret_cast<double *>(smem + L.spec);
+    T *const su = reinterpret_cast<T *>(smem + L.su);
+    unsigned char *const acc = smem + L.acc;
+    const size_t part = (size_t)ch.part_base;
+    struct Chunk {
+        T *c;
+        unsigned short *q;
+        int *off, *n;
+    };
+    auto chunk = [&](int k) {
+        unsigned char *s = smem + L.ck[k];
+        Chunk x;
+        x.c = reinterpret_cast<T *>(s);
+        s += align16((size_t)cap * sizeof(T));
+        x.q = reinterpret_cast<unsigned short *>(s);
+        s += align16((size_t)cap * 2);
+        x.off = reinterpret_cast<int *>(s);
+        x.n = reinterpret_cast<int *>(s + align16((kChunk + 1) * 4));
+        return x;
+    };
+    // the pairs of the chunk that starts at try pa, by waves w0, w0 + 1, ...: as many tries as the
+    // buffer holds (each wave takes the same prefix of the counts)
+    auto fetch = [&](const Chunk &x, int pa, int w0) {
+        if (pa >= N) return;
+        const int v = pa + lane < N ? B.cnt[part + pa + lane] : 0;
+        int tot;
+        const int pre = wave_prefix(v, lane, tot);
+        const int nf = __popcll(__ballot(pa + lane < N && pre + v <= cap));
+        if (wave == w0) {
+            x.off[lane] = pre;
+            if (lane == nf - 1) {
+                x.off[nf] = pre + v;
+                *x.n = nf;
+            }
+        }
+        for (int l = wave - w0; l < nf; l += nwv - w0) {
+            const int p = pa + l, n = __shfl(v, l, 64), o = __shfl(pre, l, 64);
+            const unsigned short *row = B.row(ch, p);
+            const T *val = B.vals(ch, 0) + pair_row(p);
+            const size_t step = pair_row(N);
+            for (int k = lane; k < n; k += 64) {
+                T s = T(0);
+                bool hit = false;
+#pragma unroll 8
+                for (int w = 0; w < nw; ++w) {
+                    const T y = val[(size_t)w * step + k];
+                    hit = hit || y != T(0) || is_neg_zero(y);
+                    s = add_(s, y);
+                }
+                x.c[o + k] = s;
+                x.q[o + k] = (unsigned short)(row[k] | (hit ? 0x8000 : 0));
+            }
+        }
+    };
+    fetch(chunk(0), 0, 0);
     for (int p = tid; p < N; p += nt) {
         double s = 0.0;
-        for (int w = 0; w < nw; ++w) s += spec[((size_t)ch.part_base + p) * nwin + w];
+        for (int w = 0; w < nw; ++w) s += B.spec[(part + p) * B.nwin + w];
         s_spec[p] = s;
         T d[DIM], u;
         com_try<T, DIM>(a, c, sw, p, d, u);
-#pragma unroll
-        for (int e = 0; e < DIM; ++e) sd[p * DIM + e] = d[e];
         su[p] = u;
         acc[p] = 0;
-        const float4 b0 = wb[(size_t)p * nwin];
-        float sx = 0.f, sy = 0.f;
-        for (int w = 0; w < nw; ++w) {
-            const float4 b = wb[(size_t)p * nwin + w];
-            sx += mi_f(b.x - b0.x, twoL, inv2L);
-            if (DIM > 1) sy += mi_f(b.y - b0.y, twoL, inv2L);
-        }
-        sx /= (float)nw;
-        sy /= (float)nw;
-        float r = 0.f;
-        for (int w = 0; w < nw; ++w) {
-            const float4 b = wb[(size_t)p * nwin + w];
-            const float dx = mi_f(b.x - b0.x, twoL, inv2L) - sx, dy = DIM > 1 ? mi_f(b.y - b0.y, twoL, inv2L) - sy : 0.f;
-            r = fmaxf(r, sqrtf(dx * dx + dy * dy) + b.z);
-        }
-        rb[p] = make_float4(b0.x + sx, b0.y + sy, r * 1.00001f, 0.f);
     }
     __syncthreads();
-    auto fshift = [&](int k, float *f) {
-        f[0] = (float)sd[k * DIM];
-        if (DIM > 1) f[1] = (float)sd[k * DIM + DIM - 1];
-    };
     int nacc = 0;
-    for (int pa = 0; pa < N;) {
-        const int nf = chunk_slots(X, pa, N, cap, kc, [&](int p, int q) {
-            if (q >= p) return false;
-            if (q < pa && !acc[q]) return false;
-            float dp[2], dq[2];
-            fshift(p, dp);
-            fshift(q, dq);
-            return bnd_near4<DIM>(rb[p], dp, rb[q], dq, h, twoL, inv2L);
-        });
-        const int total = X.misc[1];
-        for (int it = tid; it < nf * nw; it += nt) {
-            const int l = it / nw, w = it - l * nw;
-            pwb[l * 32 + w] = wb[(size_t)(pa + l) * nwin + w];
-        }
-        __syncthreads();
-        // the windows of each slot whose bounds (old or shifted) come within reach:
-        // one thread per (slot, 4 windows), q's bounds fetched together
-        for (int i = tid; i < total; i += nt) {
-            s_wm[i] = 0u;
-            s_hitf[i] = 0;
-            X.pc[i] = T(0);
-        }
-        __syncthreads();
-        const int ngrp = (nw + 3) / 4;
-        for (int it = tid; it < total * ngrp; it += nt) {
-            const int i = it / ngrp, w0 = (it - i * ngrp) * 4;
-            const int l = X.po[i], p = pa + l, q = X.pq[i];
-            float dp[2], dq[2];
-            fshift(p, dp);
-            fshift(q, dq);
-            float4 bq[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (w0 + k < nw) bq[k] = wb[(size_t)q * nwin + w0 + k];
-            unsigned bits = 0u;
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (w0 + k < nw && bnd_near4<DIM>(pwb[l * 32 + w0 + k], dp, bq[k], dq, h, twoL, inv2L))
-                    bits |= 1u << (w0 + k);
-            if (bits) atomicOr(s_wm + i, bits);
-        }
-        __syncthreads();
-        // items = (slot, window) in slot order, windows ascending within a slot
-        if (wave == 0) {
-            const int lane = tid;
-            int base = 0;
-            for (int i0 = 0; i0 < total; i0 += 64) {
-                const int i = i0 + lane;
-                const int v = i < total ? __popc(s_wm[i]) : 0;
-                int tot;
-                const int pre = wave_prefix(v, lane, tot);
-                if (i < total) s_ioff[i] = base + pre;
-                base += tot;
-            }
-            if (lane == 0) X.misc[2] = base;
-        }
-        __syncthreads();
-        const int nitems = X.misc[2];
-        for (int k0 = 0; k0 < nitems; k0 += kItemBatch) {
-            const int kn = min(kItemBatch, nitems - k0);
-            for (int kk = tid; kk < kn; kk += nt) {
-                const int k = k0 + kk;
-                int lo = 0, hi = total - 1; // the last slot whose first item is <= k
-                while (lo < hi) {
-                    const int mid = (lo + hi + 1) >> 1;
-                    if (s_ioff[mid] <= k) lo = mid;
-                    else hi = mid - 1;
-                }
-                const int i = lo;
-                unsigned wm = s_wm[i];
-                for (int r = k - s_ioff[i]; r > 0; --r) wm &= wm - 1u;
-                const int w = __ffs((int)wm) - 1;
-                const int p = pa + X.po[i], q = X.pq[i];
-                const int s0 = w * lc, m = min(lc, M - s0);
-                auto bead = [&](int t, int who, T *ro, T *rn) {
-                    const int kp = who ? q : p;
-                    int j = s0 + t;
-                    if (j >= M) j -= M;
-                    const T *r = ring + ((size_t)kp * M + j) * DIM;
-                    if constexpr (DIM == 2) {
-                        using V2 = typename std::conditional<sizeof(T) == 4, float2, double2>::type;
-                        const V2 v = *reinterpret_cast<const V2 *>(r);
-                        ro[0] = v.x;
-                        ro[1] = v.y;
-                    } else {
-                        ro[0] = r[0];
-                    }
-#pragma unroll
-                    for (int e = 0; e < DIM; ++e) rn[e] = teleport(ro[e] + sd[kp * DIM + e], P);
-                };
-                T A, Cw;
-                bool hw;
-                pair_window<T, DIM, 4>(bead, m, true, P, ch.nbins, A, Cw, hw);
-                s_cw[kk] = Cw;
-                s_hw[kk] = hw ? 1 : 0;
-            }
-            __syncthreads();
-            // each slot adds its items of this batch in window order
-            for (int i = tid; i < total; i += nt) {
-                const int b0 = max(s_ioff[i], k0), b1 = min(s_ioff[i] + __popc(s_wm[i]), k0 + kn);
-                T acc_c = X.pc[i];
-                unsigned char hf = s_hitf[i];
-                for (int k = b0; k < b1; ++k) {
-                    acc_c += s_cw[k - k0];
-                    hf |= s_hw[k - k0];
-                }
-                X.pc[i] = acc_c;
-                s_hitf[i] = hf;
-            }
-            __syncthreads();
-        }
-        for (int i = tid; i < total; i += nt)
-            if (s_hitf[i]) X.pq[i] = (unsigned short)(X.pq[i] | 0x8000);
-        __syncthreads();
-        if (tid < nf) {
-            X.spec[tid] = s_spec[pa + tid];
-            X.nb[tid] = X.off[tid] + X.cnt[tid];
-        }
-        __syncthreads();
-        if (wave == 0) {
-            const unsigned long long am = chunk_decide<T>(X, pa, nf, acc, [&](int p) { return su[p]; });
-            const int l = tid;
-            if (l < nf) acc[pa + l] = (unsigned char)((am >> l) & 1ull);
+    for (int pa = 0, k = 0; pa < N; k ^= 1) {
+        const Chunk x = chunk(k);
+        const int nf = *x.n;
+        if (wave > 0) {
+            fetch(chunk(k ^ 1), pa + nf, 1);
+        } else {
+            const unsigned long long am = chunk_decide<T>(x.q, x.c, lane < nf ? x.off[lane] : 0, lane < nf ? x.off[lane + 1] : 0,
+                                                          lane < nf ? s_spec[pa + lane] : 0.0, lane < nf ? su[pa + lane] : T(0),
+                                                          pa, nf, acc);
+            if (lane < nf) acc[pa + lane] = (unsigned char)((am >> lane) & 1ull);
             nacc += __popcll(am);
         }
         __syncthreads();
         pa += nf;
     }
-    for (int p = tid; p < N; p += nt) {
-        const size_t q = (size_t)ch.part_base + p;
-        cacc[q] = acc[p];
-#pragma unroll
-        for (int e = 0; e < DIM; ++e) cshift[q * 2 + e] = sd[p * DIM + e];
-    }
+    for (int p = tid; p < N; p += nt) cacc[part + p] = acc[p];
     if (tid == 0) {
         double *out = a.chain_meas + (size_t)c * (kNQ + kCnt);
         out[kNQ + 1] += (double)nacc;
