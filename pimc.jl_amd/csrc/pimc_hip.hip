@@ -116,7 +116,10 @@ struct pimc_ctx {
     int *d_win_all = nullptr;
     int win_seg = 0, win_maxN = 0, win_maxM = 0, win_maxell = 0, win_maxM0 = 0;
     int cap_stage = 0, cap_cspec = 0, cap_cdec = 0;   // pair-slot pools of the three kernels
-    int rows_cspec = 64, nt_cspec = 512;              // k_com_spec: particles per block, threads
+    // staging and phase-1 kernels: particles per block, threads; staging: pairs kept in LDS, candidates
+    // per chunk of tries
+    int rows_stage = 64, nt_stage = 512, rows_cspec = 64, nt_cspec = 512, keep_stage = 0, stage_cand = 0;
+    int win_nval = 1;                                 // values kept per pair slot (ComBuf::nval)
     size_t lds_stage = 0, lds_cspec = 0, lds_cdec = 0, lds_cells = 0, lds_cbnd = 0;
     int cells_wpg = 4, win_ncell = 0;                 // k_cells_win: waves per workgroup, largest cell count
     // centre-of-mass pass of the window chains (ComBuf)
@@ -675,9 +678,6 @@ template <typename T, int DIM> void launch_win_d(pimc_ctx *c, const SweepArgs &b
     w.whole = c->d_win_all + c->wg_off[g];
     const hipStream_t st = win_stream(c, g);
     if (stagger && g == 1) HIPCHK(hipStreamWaitEvent(st, stagger, 0));
-    hipLaunchKernelGGL((k_stage_win<T, DIM>), dim3((unsigned)c->win_seg, (unsigned)n), dim3(512), c->lds_stage, st,
-                       w, c->cap_stage);
-    HIPCHK(hipGetLastError());
     ComBuf<T> B{};
     B.wbnd = static_cast<float4 *>(c->d_wbnd);
     B.rbnd = static_cast<float4 *>(c->d_rbnd);
@@ -687,10 +687,14 @@ template <typename T, int DIM> void launch_win_d(pimc_ctx *c, const SweepArgs &b
     B.partner = c->d_partner;
     B.cval = static_cast<T *>(c->d_cval);
     B.nwin = c->spec_nwin;
+    B.nval = c->win_nval;
     const unsigned blk = (unsigned)((c->win_maxN + 63) / 64);
     for (const auto &[first, nb] : c->wg_batch[g]) {
         SweepArgs v = w;
         v.whole = c->d_win_all + first;
+        hipLaunchKernelGGL((k_stage_win<T, DIM>), dim3((unsigned)c->win_seg, (unsigned)nb), dim3(c->nt_stage),
+                           c->lds_stage, st, v, B, c->rows_stage, c->cap_stage, c->keep_stage, c->stage_cand);
+        HIPCHK(hipGetLastError());
         hipLaunchKernelGGL((k_com_bounds<T, DIM>), dim3(blk, (unsigned)nb), dim3(256), c->lds_cbnd, st, v, B);
         HIPCHK(hipGetLastError());
         hipLaunchKernelGGL((k_com_pairs<T, DIM>), dim3(blk, (unsigned)nb), dim3(256), 0, st, v, B);
@@ -1301,7 +1305,7 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
                 if (win) {
                     const int N = std::max(c->win_maxN, h.N), ell = std::max(c->win_maxell, h.ell);
                     const int lc = std::max(com_win_len(std::max(c->win_maxM, h.M)), 8);
-                    win = stage_lds(N, ell, h.dim, tsz, N).ck.end <= 160 * 1024 &&
+                    win = stage_lds(N, ell, h.dim, tsz, 64, N, 0).end <= 160 * 1024 &&
                           com_spec_lds(N, lc, h.dim, tsz, 64, N).end <= 160 * 1024 &&
                           com_dec_lds(N, tsz, N).end <= 160 * 1024;
                 }
@@ -1491,10 +1495,6 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
         c->d_win_all = dalloc<int>(c->win_all.size());
         if (!c->win_all.empty()) {
             HIPCHK(hipMemcpy(c->d_win_all, c->win_all.data(), sizeof(int) * c->win_all.size(), hipMemcpyHostToDevice));
-            // pools: at least N slots (one particle's partners), at most a whole chunk's, and
-            // otherwise what keeps the staging kernel within 64 KiB (two 512-thread workgroups
-            // per CU), the phase-1 kernel within 48 KiB (three) and the decision kernel (one
-            // workgroup per chain) within 128 KiB; measured on gauss_box and lattice
             const int N = c->win_maxN, ts_ = (int)ts, d = c->dim;
             const int lc = std::max(com_win_len(c->win_maxM), 8);
             auto grow = [&](auto bytes, size_t limit) {
@@ -1502,20 +1502,47 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
                 while (cap > N && bytes(cap) > limit) cap -= 64;
                 return std::max(cap, N);
             };
-            c->cap_stage = grow([&](int k) { return stage_lds(N, c->win_maxell, d, ts_, k).ck.end; }, 64 * 1024);
-            // blocks of up to 256 particles, fewer where the masks do not leave room for the pool
-            c->rows_cspec = 256;
-            while (c->rows_cspec > 64 && com_spec_lds(N, lc, d, ts_, c->rows_cspec, N).end > 120 * 1024) c->rows_cspec >>= 1;
-            c->cap_cspec = grow([&](int k) { return com_spec_lds(N, lc, d, ts_, c->rows_cspec, k).end; }, 80 * 1024);
-            if (c->cap_cspec < 4 * N) // more than half of the LDS anyway: one workgroup per CU
-                c->cap_cspec = grow([&](int k) { return com_spec_lds(N, lc, d, ts_, c->rows_cspec, k).end; }, 128 * 1024);
+            // Staging and phase-1 kernels: the largest block of particles (rows) whose expected pairs fit
+            // half of a CU's LDS, so that two 512-thread workgroups share it; where no block of 128 does,
+            // one 1024-thread workgroup a CU.  Expected pairs q < p of a row: the particles within 1.35
+            // cut-offs (the cut-off and two window radii), half of them
+            double est = 1.0;
+            for (int id : c->win_all) {
+                const ChainDev &h = c->ch[id];
+                const double r = 1.35 * h.h / (2.0 * h.L), vol = h.dim == 1 ? 2.0 * r : 3.14159265358979 * r * r;
+                est = std::max(est, 0.5 * h.N * std::min(1.0, vol));
+            }
+            auto blocks = [&](auto bytes, int &rows, int &cap, int &nt) {
+                for (size_t limit : {(size_t)80 * 1024, (size_t)158 * 1024})
+                    for (rows = std::min(1024, (N + 63) / 64 * 64); rows >= std::min(128, (N + 63) / 64 * 64);
+                         rows = rows > 128 ? (rows / 2 + 63) / 64 * 64 : 0) {
+                        cap = std::max(N, std::min(16384, (int)(1.15 * est * rows) + 64));
+                        nt = limit > 80 * 1024 ? 1024 : 512;
+                        if (bytes(rows, cap) <= limit) return limit;
+                    }
+                rows = 64;
+                cap = N;
+                nt = 1024;
+                return (size_t)160 * 1024;
+            };
+            const size_t stage_limit =
+                blocks([&](int r, int k) { return stage_lds(N, c->win_maxell, d, ts_, r, k, 0).end; }, c->rows_stage,
+                       c->cap_stage, c->nt_stage);
+            c->keep_stage = 0; // the rest of the LDS holds the window's pairs
+            for (int k = 64; k <= 16384 && stage_lds(N, c->win_maxell, d, ts_, c->rows_stage, c->cap_stage, k).end <= stage_limit; k += 64)
+                c->keep_stage = k;
+            c->stage_cand = stage_budget(N, c->win_maxell, d, ts_);
+            (void)blocks([&](int r, int k) { return com_spec_lds(N, lc, d, ts_, r, k).end; }, c->rows_cspec, c->cap_cspec,
+                         c->nt_cspec);
+            // values per pair slot: C of every centre-of-mass window, or the staging windows' pairs (a value
+            // and a partner each)
+            c->win_nval = std::max(c->spec_nwin, (int)((c->win_seg * (ts + 2) + ts - 1) / ts));
             c->cap_cdec = grow([&](int k) { return com_dec_lds(N, ts_, k).end; }, 128 * 1024);
             c->cap_meas = grow([&](int k) { return meas_win_lds(N, lc, d, ts_, k).ck.end; }, 48 * 1024);
             c->lds_meas = meas_win_lds(N, lc, d, ts_, c->cap_meas).ck.end;
             c->d_win_part = dalloc<double>(c->win_all.size() * (size_t)c->spec_nwin * 6);
-            c->lds_stage = stage_lds(N, c->win_maxell, d, ts_, c->cap_stage).ck.end;
+            c->lds_stage = stage_lds(N, c->win_maxell, d, ts_, c->rows_stage, c->cap_stage, c->keep_stage).end;
             c->lds_cspec = com_spec_lds(N, lc, d, ts_, c->rows_cspec, c->cap_cspec).end;
-            c->nt_cspec = c->lds_cspec > 80 * 1024 ? 1024 : 512;
             c->lds_cdec = com_dec_lds(N, ts_, c->cap_cdec).end;
             c->lds_cbnd = (size_t)c->spec_nwin * kBndPart * sizeof(float4);
             c->cells_wpg = 4;
@@ -1556,7 +1583,7 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
             // a time as kPairBytes holds (at least one)
             size_t slots = 0;
             for (int g = 0; g < c->n_wgroup; ++g) {
-                const size_t limit = kPairBytes / ((size_t)c->spec_nwin * ts);
+                const size_t limit = kPairBytes / ((size_t)c->win_nval * ts);
                 size_t used = 0, most = 0;
                 int first = c->wg_off[g];
                 const int end = c->wg_off[g] + c->wg_n[g];
@@ -1576,7 +1603,7 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
                 slots += most;
             }
             c->d_partner = dalloc<unsigned short>(slots);
-            HIPCHK(hipMalloc(&c->d_cval, std::max<size_t>(1, slots) * c->spec_nwin * ts));
+            HIPCHK(hipMalloc(&c->d_cval, std::max<size_t>(1, slots) * c->win_nval * ts));
             std::vector<char> has_cells(n_chains, 0);
             for (int id : c->win_ids[0]) has_cells[id] = 1;
             for (int g = 0; g < c->n_wgroup; ++g) {

@@ -122,29 +122,8 @@ __device__ __forceinline__ bool bnd_near4(float4 A, const float *da, float4 B, c
 
 // --- pair terms of one window ---
 
-// Per slice of a link pairing: squared distance test, pair potential and
-// stencil multiplicity of the query bead x (particle p) against y (particle q).
-template <typename T, int DIM> struct SliceTerm {
-    T e, mult;
-    bool in;
-    __device__ __forceinline__ void eval(const T *x, const T *y, const Prm<T> &P, int nbins)
-    {
-        const T d2 = dist2<T, DIM>(x, y, P);
-        in = d2 <= P.h2;
-        e = vpair_r2(d2, P);
-        mult = (nbins >= 3) ? T(1) : stencil_mult<T, DIM>(x, y, P, nbins);
-    }
-    // lnU of the link from this slice (the query slice) to the next: the term a
-    // neighbour adds in interaction_action! (src/updates/helper.jl:326-346), 0 for a
-    // bead outside the cut-off (not among find_nns's neighbours)
-    __device__ __forceinline__ T link(const SliceTerm &next, T ctau) const
-    {
-        return in ? mult * (ctau * (e + next.e)) : T(0);
-    }
-};
-
-// Sums and products that keep their roundings: pair_window's forms, whatever
-// code surrounds them.
+// Sums and products of the pair terms keep their own roundings, whatever code
+// surrounds them.
 template <typename T> __device__ __forceinline__ T add_(T x, T y)
 {
 #pragma clang fp contract(off)
@@ -176,64 +155,6 @@ template <typename T, int DIM> __device__ __forceinline__ T dist2_min(const T *x
     if (DIM == 1) return d0 * d0;
     const T d1 = mindist_min(x[DIM - 1], y[DIM - 1], P);
     return fma_(d0, d0, d1 * d1);
-}
-
-// A(p, q) and, for q < p (back), C(p, q) over the links 0..m-1 of one window.
-// bead(t, who, ro, rn): old and new bead of particle p (who 0) or q (who 1) at
-// window slice t.  Slices are fetched B at a time before any is used (B > 1
-// lets loads from HBM overlap).  ENDS: the old and new beads coincide at slices
-// 0 and m (staging), so one pairing is evaluated there.  hit: some pairing has
-// a term within the cut-off.
-template <typename T, int DIM, int B, bool ENDS = false, typename BeadFn>
-__device__ __forceinline__ void pair_window(BeadFn bead, int m, bool back, const Prm<T> &P, int nbins, T &A, T &C,
-                                            bool &hit)
-{
-    const T ctau = T(-0.5) * P.tau;
-    SliceTerm<T, DIM> oo, no, on, nn;
-    A = T(0);
-    C = T(0);
-    bool any = false;
-    for (int t0 = 0; t0 <= m; t0 += B) {
-        T po[B][DIM], pn[B][DIM], qo[B][DIM], qn[B][DIM];
-#pragma unroll
-        for (int k = 0; k < B; ++k)
-            if (t0 + k <= m) {
-                bead(t0 + k, 0, po[k], pn[k]);
-                bead(t0 + k, 1, qo[k], qn[k]);
-            }
-#pragma unroll
-        for (int k = 0; k < B; ++k) {
-            const int t = t0 + k;
-            if (t > m) break;
-            SliceTerm<T, DIM> oo1, no1, on1, nn1;
-            oo1.eval(po[k], qo[k], P, nbins);
-            if (ENDS && (t == 0 || t == m)) {
-                no1 = oo1;
-                on1 = oo1;
-                nn1 = oo1;
-            } else {
-                no1.eval(pn[k], qo[k], P, nbins);
-                if (back) {
-                    on1.eval(po[k], qn[k], P, nbins);
-                    nn1.eval(pn[k], qn[k], P, nbins);
-                }
-            }
-            if (t > 0) {
-                const T too = oo.link(oo1, ctau), tno = no.link(no1, ctau);
-                const T a = tno - too;
-                A += a;
-                if (back) C += (nn.link(nn1, ctau) - on.link(on1, ctau)) - a;
-            }
-            if (t < m) {
-                any = any || oo1.in || no1.in || (back && (on1.in || nn1.in));
-                oo = oo1;
-                no = no1;
-                on = on1;
-                nn = nn1;
-            }
-        }
-    }
-    hit = any;
 }
 
 // --- ordered pair lists of a chunk of particles ---
@@ -389,6 +310,32 @@ __device__ inline void grid_build(WinGrid &G, int N, float h, float twoL, float 
     __syncthreads();
 }
 
+// The members of particle p's stencil, flattened over the lanes of a wave.
+template <int DIM, typename Visit> __device__ __forceinline__ void grid_visit(const WinGrid &G, int p, int lane, Visit visit)
+{
+    const int ng = G.ng;
+    constexpr int NS = DIM == 1 ? 3 : 9;
+    const int pc = G.pcell[p];
+    const int ix = DIM == 1 ? pc : pc % ng, iy = DIM == 1 ? 0 : pc / ng;
+    int b[NS], pre[NS + 1];
+    pre[0] = 0;
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        int cx = ix + k % 3 - 1, cy = iy + (DIM == 1 ? 0 : k / 3 - 1);
+        cx += cx < 0 ? ng : (cx >= ng ? -ng : 0);
+        cy += cy < 0 ? ng : (cy >= ng ? -ng : 0);
+        const int cc = cx + ng * cy;
+        b[k] = cc ? G.start[cc - 1] : 0;
+        pre[k + 1] = pre[k] + G.start[cc] - b[k];
+    }
+    for (int i = lane; i < pre[NS]; i += 64) {
+        int at = b[0] + i;
+#pragma unroll
+        for (int k = 1; k < NS; ++k) at = i >= pre[k] ? b[k] + (i - pre[k]) : at;
+        visit((int)G.mem[at]);
+    }
+}
+
 // Slots of the chunk's particles pa, pa + 1, ... (at most kc <= kChunk): for
 // each the partners q with cand(p, q), by index.  Fills as many particles as
 // the pool holds (at least one: cap >= N).  Returns the number of particles filled; X.misc[1] is the
@@ -402,31 +349,13 @@ __device__ inline int chunk_slots(ChunkPtr<T> &X, int pa, int N, int cap, int kc
     if (G && G->ng > 0) {
         // candidates from the grid stencil (one wave per particle, the stencil's members
         // flattened over the lanes), set as bits of the particle's mask
-        const int ng = G->ng;
-        constexpr int NS = DIM == 1 ? 3 : 9;
         for (int i = tid; i < nc * nq; i += nt) X.mask[i] = 0ull;
         __syncthreads();
         for (int l = wave; l < nc; l += nwv) {
-            const int p = pa + l, pc = G->pcell[p];
-            const int ix = DIM == 1 ? pc : pc % ng, iy = DIM == 1 ? 0 : pc / ng;
-            int b[NS], pre[NS + 1];
-            pre[0] = 0;
-#pragma unroll
-            for (int k = 0; k < NS; ++k) {
-                int cx = ix + k % 3 - 1, cy = iy + (DIM == 1 ? 0 : k / 3 - 1);
-                cx += cx < 0 ? ng : (cx >= ng ? -ng : 0);
-                cy += cy < 0 ? ng : (cy >= ng ? -ng : 0);
-                const int cc = cx + ng * cy;
-                b[k] = cc ? G->start[cc - 1] : 0;
-                pre[k + 1] = pre[k] + G->start[cc] - b[k];
-            }
-            for (int i = lane; i < pre[NS]; i += 64) {
-                int at = b[0] + i;
-#pragma unroll
-                for (int k = 1; k < NS; ++k) at = i >= pre[k] ? b[k] + (i - pre[k]) : at;
-                const int q = G->mem[at];
+            const int p = pa + l;
+            grid_visit<DIM>(*G, p, lane, [&](int q) {
                 if (cand(p, q)) atomicOr(X.mask + l * nq + (q >> 6), 1ull << (q & 63));
-            }
+            });
         }
         __syncthreads();
         for (int l = tid; l < nc; l += nt) {
@@ -482,8 +411,8 @@ __device__ inline int chunk_slots(ChunkPtr<T> &X, int pa, int N, int cap, int kc
 }
 
 // Decisions of the chunk's tries pa .. pa + nf - 1 in index order (one wave,
-// lane l decides try pa + l).  Slots o0 .. o1 of pq, pc hold the try's earlier
-// partners by index (hit flag in bit 15) with their C values, sp its sum against
+// lane l decides try pa + l).  pq(i), pc(i), i in o0 .. o1, are the try's earlier
+// partners by index (hit flag in bit 15) and their C values, sp its sum against
 // the configuration at the start, u its uniform; acc[q] holds the decisions of
 // the tries before the chunk.  A try waits for its earlier partners inside the
 // chunk that have a term within the cut-off (the others add exactly zero).  Each
@@ -491,9 +420,9 @@ __device__ inline int chunk_slots(ChunkPtr<T> &X, int pa, int N, int cap, int kc
 // partners before the chunk in index order, then the partners inside the chunk as
 // they are accepted (by round, in index order within a round), a fixed order.
 // Returns the acceptance mask.
-template <typename T>
-__device__ inline unsigned long long chunk_decide(const unsigned short *pq, const T *pc, int o0, int o1, double sp, T u,
-                                                  int pa, int nf, const unsigned char *acc)
+template <typename T, typename Q, typename C>
+__device__ inline unsigned long long chunk_decide(Q pq, C pc, int o0, int o1, double sp, T u, int pa, int nf,
+                                                  const unsigned char *acc)
 {
     const int l = threadIdx.x & 63;
     const bool in = l < nf;
@@ -501,9 +430,9 @@ __device__ inline unsigned long long chunk_decide(const unsigned short *pq, cons
     unsigned long long dep = 0ull, pm = 0ull; // in-chunk partners with a term within the cut-off, all
     int si = o1;                              // first in-chunk partner's slot
     for (int i = o0; i < o1; ++i) {
-        const int qq = pq[i], q = qq & 0x7fff;
+        const int qq = pq(i), q = qq & 0x7fff;
         if (q < pa) {
-            if (acc[q]) tot += pc[i];
+            if (acc[q]) tot += pc(i);
         } else {
             if (si == o1) si = i;
             pm |= 1ull << (q - pa);
@@ -526,7 +455,7 @@ __device__ inline unsigned long long chunk_decide(const unsigned short *pq, cons
             while (b) {
                 const int k = __ffsll((long long)b) - 1;
                 b &= b - 1;
-                tot += pc[si + __popcll(pm & ((1ull << k) - 1ull))];
+                tot += pc(si + __popcll(pm & ((1ull << k) - 1ull)));
             }
         }
     }
@@ -543,45 +472,197 @@ __global__ void k_clear_chain_meas(double *chain_meas, const int *ids, int n)
     for (int k = threadIdx.x; k < kNQ + kCnt; k += blockDim.x) o[k] = 0.0;
 }
 
+// Index of pair (p, q = 0) among the pairs p > q of a chain.
+__host__ __device__ __forceinline__ size_t pair_row(int p) { return (size_t)p * (size_t)(p - 1) / 2; }
+
+// Buffers of the centre-of-mass kernels.  Per particle (window chains only, by
+// part_base) wbnd[. * nwin + w] bounds its old beads in window w, rbnd its old
+// ring, shift/unif hold its try, cnt the listed partners; per pair slot
+// (ChainDev::pair_off + pair_row(p) + k, the k-th listed partner of p by index)
+// partner; per window and slot (at nval times the chain's pair offset)
+// cval: C of the window, with +0 for "no term within the cut-off" (a value of
+// zero with one is stored as -0).  The staging kernel keeps the pairs that do not
+// fit its LDS in cval, before the centre-of-mass pass of the sweep fills it.
+template <typename T> struct ComBuf {
+    float4 *wbnd, *rbnd;
+    T *shift;
+    double *spec; // [particle * nwin + w]: the window's Delta V + sum_q A
+    int *cnt;
+    unsigned short *partner;
+    T *cval;
+    int nwin, nval; // windows of a particle; values kept per pair slot
+    __device__ __forceinline__ unsigned short *row(const ChainDev &ch, int p) const
+    {
+        return partner + ch.pair_off + pair_row(p);
+    }
+    __device__ __forceinline__ T *vals(const ChainDev &ch, int w) const
+    {
+        return cval + (size_t)ch.pair_off * nval + (size_t)w * pair_row(ch.N);
+    }
+};
+
+// A(p, q), A(q, p) and C(p, q) of one pair over the links 0 .. m - 1 of a window,
+// the pairings of old (o) and new (n) beads each evaluated once for both
+// particles.  A link's term is the one a neighbour adds in interaction_action!
+// (src/updates/helper.jl:326-346), from the link's first slice, 0 for a bead
+// outside the cut-off there (not among find_nns's neighbours).  bead(t, who, ro,
+// rn): old and new bead of particle p (who 0) or q (who 1) at window slice t.
+// hit: some pairing has a term within the cut-off.  MULT: chains with nbins < 3, whose terms carry a
+// stencil multiplicity.  ENDS: the old and new beads coincide at slices 0 and m
+// (staging), so one pairing is evaluated there.
+template <typename T, int DIM, bool MULT, bool ENDS = false, typename BeadFn>
+__device__ __forceinline__ void pair_window_both(BeadFn bead, int m, const Prm<T> &P, int nbins, T &Apq, T &Aqp, T &C,
+                                                 bool &hit)
+{
+    const T ctau = T(-0.5) * P.tau;
+    T e0[4], u0[4]; // the previous slice's pair potential and multiplicity: oo, no, on, nn
+    bool in0[4];
+    Apq = Aqp = C = T(0);
+    hit = false;
+    for (int t = 0; t <= m; ++t) {
+        T po[DIM], pn[DIM], qo[DIM], qn[DIM];
+        bead(t, 0, po, pn);
+        bead(t, 1, qo, qn);
+        const T *x[4] = {po, pn, po, pn}, *y[4] = {qo, qo, qn, qn};
+        T e[4], u[4], tl[4];
+        bool in[4];
+        auto eval = [&](int k) {
+            const T d2 = dist2_min<T, DIM>(x[k], y[k], P);
+            in[k] = d2 <= P.h2;
+            e[k] = vpair_r2(d2, P);
+            u[k] = MULT ? stencil_mult<T, DIM>(x[k], y[k], P, nbins) : T(1);
+        };
+        eval(0);
+        if (ENDS && (t == 0 || t == m)) {
+#pragma unroll
+            for (int k = 1; k < 4; ++k) {
+                in[k] = in[0];
+                e[k] = e[0];
+                u[k] = u[0];
+            }
+        } else {
+#pragma unroll
+            for (int k = 1; k < 4; ++k) eval(k);
+        }
+        if (t > 0) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) tl[k] = in0[k] ? link_term<MULT>(u0[k], ctau, e0[k], e[k]) : T(0);
+            const T a1 = sub_(tl[1], tl[0]);
+            Apq = add_(Apq, a1);
+            Aqp = add_(Aqp, sub_(tl[2], tl[0]));
+            C = add_(C, sub_(sub_(tl[3], tl[2]), a1));
+        }
+        if (t < m) hit = hit || in[0] || in[1] || in[2] || in[3];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            e0[k] = e[k];
+            in0[k] = in[k];
+            if (MULT) u0[k] = u[k];
+        }
+    }
+}
+
 // --- staging ---
 
+// Candidate partners (both sides) that one chunk of tries may have together: a
+// chunk ends where its tries would exceed it.  A try's sum takes the partners of
+// earlier chunks by index and those of its own chunk by round, so the chunk
+// boundaries are part of the order of the sums; this rule (what fitted 64 KiB of
+// LDS beside the window's beads when the pairs of a chunk were held for both
+// sides) keeps them where they were.
+inline int stage_budget(int N, int ell, int dim, int tsize)
+{
+    size_t o = 0;
+    auto take = [&](size_t bytes) { o = align16(o + bytes); };
+    take((size_t)(ell + 1) * N * dim * tsize);
+    take((size_t)(ell > 1 ? ell - 1 : 1) * N * dim * tsize);
+    take((size_t)N * 16);
+    take((size_t)N * tsize);
+    take((size_t)N * tsize);
+    take((size_t)N);
+    o = grid_lds(o, N, dim).end;
+    const size_t fixed = o;
+    auto bytes = [&](int cap) { return chunk_lds(fixed, N, cap, tsize, 2).end; };
+    int cap = std::min(8192, kChunk * std::max(1, N - 1));
+    while (cap > N && bytes(cap) > 64 * 1024) cap -= 64;
+    return std::max(cap, N);
+}
+
 // LDS of k_stage_win: old beads of the window's ell + 1 slices, new interior
-// beads, bounds, Delta V and Metropolis uniform per particle, decisions, then
-// the chunk machinery with pool capacity cap.
+// beads, bounds, sums, decisions, grid; masks of a block of R rows
+// (partners q < p in words of 64, and each particle's rows), the block's pool of
+// cap pairs (row and the two A values), then the window's pairs by row: partner
+// with the hit flag in bit 15 and C, the first `keep` of them here and the rest
+// in memory.
 struct StageLds {
-    size_t ob, nb, bnd, dv, su, acc;
+    size_t ob, nb, bnd, sp, acc, ncand, off, cmask, coff, misc, prow, pa, pb, pq, pc, end;
     GridLds gr;
-    ChunkLds ck;
 };
-__host__ __device__ inline StageLds stage_lds(int N, int ell, int dim, int tsize, int cap)
+__host__ __device__ inline StageLds stage_lds(int N, int ell, int dim, int tsize, int R, int cap, int keep)
 {
     StageLds L;
     size_t o = 0;
-    L.ob = o;
-    o = align16(o + (size_t)(ell + 1) * N * dim * tsize);
-    L.nb = o;
-    o = align16(o + (size_t)(ell > 1 ? ell - 1 : 1) * N * dim * tsize);
-    L.bnd = o;
-    o = align16(o + (size_t)N * 16);
-    L.dv = o;
-    o = align16(o + (size_t)N * tsize);
-    L.su = o;
-    o = align16(o + (size_t)N * tsize);
-    L.acc = o;
-    o = align16(o + (size_t)N);
+    auto take = [&](size_t bytes) {
+        const size_t at = o;
+        o = align16(o + bytes);
+        return at;
+    };
+    L.ob = take((size_t)(ell + 1) * N * dim * tsize);
+    L.nb = take((size_t)(ell > 1 ? ell - 1 : 1) * N * dim * tsize);
+    L.bnd = take((size_t)N * 16);
+    L.sp = take((size_t)N * 8);
+    L.acc = take((size_t)N);
+    L.ncand = take((size_t)N * 2);
+    L.off = take((size_t)(N + 1) * 4);
     L.gr = grid_lds(o, N, dim);
-    L.ck = chunk_lds(L.gr.end, N, cap, tsize, 2);
+    o = L.gr.end;
+    L.cmask = take((size_t)N * (R / 64) * 8);
+    L.coff = take((size_t)N * 2);
+    L.misc = take(16);
+    L.prow = take((size_t)cap * 2);
+    const size_t rows = (size_t)R * ((N + 63) / 64) * 8, vals = (size_t)cap * tsize;
+    L.pa = take(rows > vals ? rows : vals); // the row masks, then the A(p, q)
+    L.pb = take(vals);
+    L.pq = take((size_t)keep * 2);
+    L.pc = take((size_t)keep * tsize);
+    L.end = o;
     return L;
 }
 
+// The pairs of one staging window by row: the first `keep` in LDS, the others in
+// the window's part of the pair buffer (T values of all windows, then partners).
+template <typename T> struct StagePairs {
+    T *lc, *gc;
+    unsigned short *lq, *gq;
+    int keep;
+    __device__ __forceinline__ void put(int i, int q, T c) const
+    {
+        if (i < keep) {
+            lq[i] = (unsigned short)q;
+            lc[i] = c;
+        } else {
+            gq[i] = (unsigned short)q;
+            gc[i] = c;
+        }
+    }
+    __device__ __forceinline__ int q(int i) const { return i < keep ? lq[i] : gq[i]; }
+    __device__ __forceinline__ T c(int i) const { return i < keep ? lc[i] : gc[i]; }
+};
+
 // One staging window of one chain per workgroup: grid (windows, chains of the
-// list a.whole), one sweep (a.rs->sweep + a.sweep_off).
-template <typename T, int DIM> __global__ void __launch_bounds__(512) k_stage_win(SweepArgs a, int cap)
+// list a.whole), one sweep (a.rs->sweep + a.sweep_off).  The rows (particles) are
+// taken in blocks of at most R whose pairs q < p in reach fit the pool; each pair
+// is evaluated once, for A(p, q), A(q, p) and C(p, q), one pair per thread.  When
+// every pair is done the tries are decided chunk by chunk.  Pair terms are VALU
+// work (four pairings a slice); two workgroups share a CU, so one's decisions,
+// a serial chain, run beside the other's pairs.
+template <typename T, int DIM>
+__global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, int R, int cap, int keep, int budget)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const int c = a.whole[blockIdx.y];
     const ChainDev ch = a.chains[c];
-    const int w = blockIdx.x, tid = threadIdx.x, nt = blockDim.x, wave = tid >> 6;
+    const int w = blockIdx.x, tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nwv = nt >> 6;
     const int M = ch.M, N = ch.N, ell = ch.ell;
     if (w >= ch.nseg) return;
     const int m = min(ell, M - w * ell); // links of this window
@@ -599,14 +680,25 @@ template <typename T, int DIM> __global__ void __launch_bounds__(512) k_stage_wi
     if (s0 >= M) s0 -= M;
     auto slice = [&](int t) { const int j = s0 + t; return j >= M ? j - M : j; };
 
-    const StageLds L = stage_lds(N, ell, DIM, (int)sizeof(T), cap);
+    const StageLds L = stage_lds(N, ell, DIM, (int)sizeof(T), R, cap, keep);
     T *ob = reinterpret_cast<T *>(smem + L.ob); // [t][k][d], t = 0..m
     T *nb = reinterpret_cast<T *>(smem + L.nb); // [t - 1][k][d], t = 1..m-1
     float4 *bnd = reinterpret_cast<float4 *>(smem + L.bnd);
-    T *dvs = reinterpret_cast<T *>(smem + L.dv);
-    T *su = reinterpret_cast<T *>(smem + L.su);
+    double *const sp = reinterpret_cast<double *>(smem + L.sp);
     unsigned char *acc = smem + L.acc;
-    ChunkPtr<T> X(smem, L.ck);
+    unsigned short *const ncand = reinterpret_cast<unsigned short *>(smem + L.ncand);
+    int *const poff = reinterpret_cast<int *>(smem + L.off);
+    unsigned long long *const rmask = reinterpret_cast<unsigned long long *>(smem + L.pa);
+    unsigned long long *const cmask = reinterpret_cast<unsigned long long *>(smem + L.cmask);
+    unsigned short *const coff = reinterpret_cast<unsigned short *>(smem + L.coff);
+    int *const misc = reinterpret_cast<int *>(smem + L.misc);
+    unsigned short *const prow = reinterpret_cast<unsigned short *>(smem + L.prow);
+    T *const pa_ = reinterpret_cast<T *>(smem + L.pa), *const pb_ = reinterpret_cast<T *>(smem + L.pb);
+    const size_t tri = pair_row(N);
+    T *const gval = B.vals(ch, 0);
+    const StagePairs<T> S{reinterpret_cast<T *>(smem + L.pc), gval + (size_t)w * tri,
+                          reinterpret_cast<unsigned short *>(smem + L.pq),
+                          reinterpret_cast<unsigned short *>(gval + (size_t)ch.nseg * tri) + (size_t)w * tri, keep};
 
     T *const gpath = reinterpret_cast<T *>(a.pos) + ch.pos_off;
     for (int t = 0; t <= m; ++t) {
@@ -678,10 +770,11 @@ template <typename T, int DIM> __global__ void __launch_bounds__(512) k_stage_wi
             r2 = fmaxf(r2, d2);
         }
         bnd[p] = make_float4(ref[0] + mean[0], DIM > 1 ? ref[DIM - 1] + mean[DIM - 1] : 0.f, sqrtf(r2), 0.f);
-        dvs[p] = dv;
-        su[p] = Uniform<T>::get(draw(a.seed, (uint32_t)(p * M + s0), sw, (uint32_t)c, kLevyAccept).x);
+        sp[p] = (double)dv;
         acc[p] = 0;
+        ncand[p] = 0;
     }
+    if (tid == 0) poff[0] = 0;
     __syncthreads();
 
     const float h = (float)ch.h, twoL = (float)(2.0 * ch.L), inv2L = 1.0f / twoL;
@@ -704,47 +797,142 @@ template <typename T, int DIM> __global__ void __launch_bounds__(512) k_stage_wi
         y = b.y;
         r = b.z;
     });
-    int lacc = 0;
+    auto near = [&](int p, int q) {
+        const float4 A = bnd[p], Bq = bnd[q];
+        return bnd_near<DIM>(A.x, A.y, A.z, Bq.x, Bq.y, Bq.z, h, twoL, inv2L);
+    };
+    const int nq = (N + 63) / 64, nc = R / 64; // words of a row mask, of a column mask
     for (int pa = 0; pa < N;) {
-        const int nf = chunk_slots<DIM>(X, pa, N, cap, kChunk, [&](int p, int q) {
-            if (q == p) return false;
-            const float4 A = bnd[p], B = bnd[q];
-            return bnd_near<DIM>(A.x, A.y, A.z, B.x, B.y, B.z, h, twoL, inv2L);
-        }, &G);
-        const int total = X.misc[1];
-        for (int i = tid; i < total; i += nt) {
-            const int p = pa + X.po[i], q = X.pq[i];
-            T A, C;
-            bool hit;
-            pair_window<T, DIM, 1, true>(bead(p, q), m, q < p, P, ch.nbins, A, C, hit);
-            X.pa[i] = A;
-            X.pc[i] = C;
-            if (q < p && hit) X.pq[i] = (unsigned short)(q | 0x8000);
-        }
-        __syncthreads();
-        if (tid < nf) {
-            const int p = pa + tid, o0 = X.off[tid], o1 = o0 + X.cnt[tid];
-            double sp = (double)dvs[p];
-            int e = o1;
-            for (int i = o0; i < o1; ++i) {
-                sp += (double)X.pa[i];
-                if (e == o1 && (X.pq[i] & 0x7fff) > p) e = i;
+        const int nr = min(R, N - pa), base = poff[pa];
+        for (int i = tid; i < N * nc; i += nt) cmask[i] = 0ull;
+        // partners q < p in reach of each row
+        if (G.ng > 0) {
+            for (int i = tid; i < nr * nq; i += nt) rmask[i] = 0ull;
+            __syncthreads();
+            for (int l = wave; l < nr; l += nwv) {
+                const int p = pa + l;
+                grid_visit<DIM>(G, p, lane, [&](int q) {
+                    if (q < p && near(p, q)) atomicOr(rmask + (size_t)l * nq + (q >> 6), 1ull << (q & 63));
+                });
             }
-            X.spec[tid] = sp;
-            X.nb[tid] = e;
+            __syncthreads();
+            for (int l = tid; l < nr; l += nt) {
+                int cnt = 0;
+                for (int k = 0; k < nq; ++k) cnt += __popcll(rmask[(size_t)l * nq + k]);
+                poff[pa + l + 1] = cnt;
+            }
+        } else {
+            for (int l = wave; l < nr; l += nwv) {
+                const int p = pa + l;
+                int cnt = 0;
+                for (int q0 = 0; q0 < p; q0 += 64) {
+                    const int q = q0 + lane;
+                    const unsigned long long bal = __ballot(q < p && near(p, q));
+                    if (lane == 0) rmask[(size_t)l * nq + (q0 >> 6)] = bal;
+                    cnt += __popcll(bal);
+                }
+                if (lane == 0) poff[p + 1] = cnt;
+            }
         }
         __syncthreads();
-        if (wave == 0) {
-            const int l = tid;
-            const bool in = l < nf;
-            const unsigned long long am = chunk_decide<T>(X.pq, X.pc, in ? X.off[l] : 0, in ? X.nb[l] : 0, in ? X.spec[l] : 0.0,
-                                                          in ? su[pa + l] : T(0), pa, nf, acc);
-            if (l < nf) acc[pa + l] = (unsigned char)((am >> l) & 1ull);
-            lacc += __popcll(am);
+        if (wave == 0) { // prefix; the rows whose pairs fit the pool
+            int sum = 0, nf = 0;
+            for (int l0 = 0; l0 < nr; l0 += 64) {
+                const int l = l0 + lane, v = l < nr ? poff[pa + l + 1] : 0;
+                int tot;
+                const int pre = wave_prefix(v, lane, tot);
+                const bool fits = l < nr && sum + pre + v <= cap;
+                if (fits) {
+                    poff[pa + l + 1] = base + sum + pre + v;
+                    ncand[pa + l] = (unsigned short)(ncand[pa + l] + v);
+                }
+                nf += __popcll(__ballot(fits));
+                sum += tot;
+            }
+            if (lane == 0) misc[0] = nf;
+        }
+        __syncthreads();
+        const int nf = misc[0], total = poff[pa + nf] - base;
+        for (int it = tid; it < nf * nq; it += nt) {
+            const int l = it / nq, wd = it - l * nq;
+            if (wd * 64 >= pa + l) continue;
+            const unsigned long long *mk = rmask + (size_t)l * nq;
+            int s = poff[pa + l] - base;
+            for (int k = 0; k < wd; ++k) s += __popcll(mk[k]);
+            unsigned long long b = mk[wd];
+            while (b) {
+                const int q = wd * 64 + __ffsll((long long)b) - 1;
+                b &= b - 1;
+                prow[s] = (unsigned short)l;
+                S.put(base + s, q, T(0));
+                atomicOr(cmask + (size_t)q * nc + (l >> 6), 1ull << (l & 63));
+                ++s;
+            }
+        }
+        __syncthreads();
+        if (wave == 0) { // where each particle's rows start
+            int sum = 0;
+            for (int q0 = 0; q0 < N; q0 += 64) {
+                const int q = q0 + lane;
+                int v = 0, tot;
+                if (q < N)
+                    for (int k = 0; k < nc; ++k) v += __popcll(cmask[(size_t)q * nc + k]);
+                const int pre = wave_prefix(v, lane, tot);
+                if (q < N) {
+                    coff[q] = (unsigned short)(sum + pre);
+                    ncand[q] = (unsigned short)(ncand[q] + v);
+                }
+                sum += tot;
+            }
+        }
+        __syncthreads();
+        for (int i = tid; i < total; i += nt) {
+            const int l = prow[i], p = pa + l, q = S.q(base + i);
+            T Apq, Aqp, C;
+            bool hit;
+            if (ch.nbins >= 3) pair_window_both<T, DIM, false, true>(bead(p, q), m, P, ch.nbins, Apq, Aqp, C, hit);
+            else pair_window_both<T, DIM, true, true>(bead(p, q), m, P, ch.nbins, Apq, Aqp, C, hit);
+            int at = coff[q];
+            for (int k = 0; k < (l >> 6); ++k) at += __popcll(cmask[(size_t)q * nc + k]);
+            at += __popcll(cmask[(size_t)q * nc + (l >> 6)] & ((1ull << (l & 63)) - 1ull));
+            pa_[i] = Apq;
+            pb_[at] = Aqp;
+            S.put(base + i, hit ? q | 0x8000 : q, C);
+        }
+        __syncthreads();
+        for (int x = tid; x < N; x += nt) { // partners by index: the particle's own row, then the rows that name it
+            double s = sp[x];
+            if (x >= pa && x < pa + nf)
+                for (int i = poff[x] - base; i < poff[x + 1] - base; ++i) s += (double)pa_[i];
+            int n = 0;
+            for (int k = 0; k < nc; ++k) n += __popcll(cmask[(size_t)x * nc + k]);
+            for (int i = coff[x]; i < coff[x] + n; ++i) s += (double)pb_[i];
+            sp[x] = s;
         }
         __syncthreads();
         pa += nf;
     }
+    // decisions, chunk by chunk, by one wave
+    if (wave == 0) {
+        int lacc = 0;
+        for (int pa = 0; pa < N;) {
+            const int p = pa + lane, v = p < N ? (int)ncand[p] : 0;
+            int tot;
+            const int pre = wave_prefix(v, lane, tot);
+            const int nf = __popcll(__ballot(p < N && pre + v <= budget));
+            const bool in = lane < nf;
+            const T u = Uniform<T>::get(draw(a.seed, (uint32_t)(p * M + s0), sw, (uint32_t)c, kLevyAccept).x);
+            const unsigned long long am = chunk_decide<T>([&](int i) { return S.q(i); }, [&](int i) { return S.c(i); },
+                                                          in ? poff[p] : 0, in ? poff[p + 1] : 0, in ? sp[p] : 0.0, u,
+                                                          pa, nf, acc);
+            if (in) acc[p] = (unsigned char)((am >> lane) & 1ull);
+            __builtin_amdgcn_wave_barrier(); // the next chunk reads the decisions
+            lacc += __popcll(am);
+            pa += nf;
+        }
+        if (lane == 0) atomicAdd(a.chain_meas + (size_t)c * (kNQ + kCnt) + kNQ, (double)lacc);
+    }
+    __syncthreads();
     // accepted proposals to HBM
     for (int i = 1; i < m; ++i) {
         T *dst = gpath + (size_t)slice(i) * N * DIM;
@@ -755,7 +943,6 @@ template <typename T, int DIM> __global__ void __launch_bounds__(512) k_stage_wi
                 for (int e = 0; e < DIM; ++e) dst[k * DIM + e] = src[k * DIM + e];
             }
     }
-    if (tid == 0) atomicAdd(a.chain_meas + (size_t)c * (kNQ + kCnt) + kNQ, (double)lacc);
 }
 
 // --- centre of mass ---
@@ -770,34 +957,6 @@ __device__ __forceinline__ void com_try(const SweepArgs &a, int c, uint32_t sw, 
     if (DIM > 1) d[1] = s2 * (Uniform<T>::get(y.y) - T(0.5));
     u = Uniform<T>::get(y.z);
 }
-
-// Index of pair (p, q = 0) among the pairs p > q of a chain.
-__host__ __device__ __forceinline__ size_t pair_row(int p) { return (size_t)p * (size_t)(p - 1) / 2; }
-
-// Buffers of the centre-of-mass kernels.  Per particle (window chains only, by
-// part_base) wbnd[. * nwin + w] bounds its old beads in window w, rbnd its old
-// ring, shift/unif hold its try, cnt the listed partners; per pair slot
-// (ChainDev::pair_off + pair_row(p) + k, the k-th listed partner of p by index)
-// partner; per window and slot (at nwin times the chain's pair offset)
-// cval: C of the window, with +0 for "no term within the cut-off" (a value of
-// zero with one is stored as -0).
-template <typename T> struct ComBuf {
-    float4 *wbnd, *rbnd;
-    T *shift;
-    double *spec; // [particle * nwin + w]: the window's Delta V + sum_q A
-    int *cnt;
-    unsigned short *partner;
-    T *cval;
-    int nwin;
-    __device__ __forceinline__ unsigned short *row(const ChainDev &ch, int p) const
-    {
-        return partner + ch.pair_off + pair_row(p);
-    }
-    __device__ __forceinline__ T *vals(const ChainDev &ch, int w) const
-    {
-        return cval + (size_t)ch.pair_off * nwin + (size_t)w * pair_row(ch.N);
-    }
-};
 
 // Whether the bounds of two particles come within reach in one of the four
 // pairings of old and shifted beads.
@@ -934,7 +1093,7 @@ template <typename T, int DIM> __global__ void __launch_bounds__(256) k_com_pair
 // reach (words of 64 list entries) and of each particle's rows (words of 64
 // rows), then the pool: row, list index, partner and the two A values.
 struct ComSpecLds {
-    size_t ob, sd, sp, rmask, roff, cmask, coff, misc, prow, pk, pq, pa, pb, end;
+    size_t ob, sd, sp, roff, cmask, coff, misc, prow, pk, pq, pa, pb, end;
 };
 __host__ __device__ inline ComSpecLds com_spec_lds(int N, int lc, int dim, int tsize, int R, int cap)
 {
@@ -949,63 +1108,18 @@ __host__ __device__ inline ComSpecLds com_spec_lds(int N, int lc, int dim, int t
     L.ob = take((size_t)(lc + 1) * N * dim * tsize);
     L.sd = take((size_t)N * dim * tsize);
     L.sp = take((size_t)N * 8);
-    L.rmask = take((size_t)R * nq * 8);
     L.roff = take((size_t)(R + 1) * 4);
     L.cmask = take((size_t)N * (R / 64) * 8);
     L.coff = take((size_t)N * 2);
     L.misc = take(16);
-    L.prow = take((size_t)cap);
+    L.prow = take((size_t)cap * 2);
     L.pk = take((size_t)cap * 2);
     L.pq = take((size_t)cap * 2);
-    L.pa = take((size_t)cap * tsize);
-    L.pb = take((size_t)cap * tsize);
+    const size_t rows = (size_t)R * nq * 8, vals = (size_t)cap * tsize;
+    L.pa = take(rows > vals ? rows : vals); // the row masks, then the A(p, q)
+    L.pb = take(vals);
     L.end = o;
     return L;
-}
-
-// A(p, q), A(q, p) and C(p, q) of one pair over the links 0 .. m - 1 of a window:
-// pair_window's terms, the pairings of old (o) and new (n) beads each evaluated
-// once for both particles.  MULT: chains with nbins < 3, whose terms carry a
-// stencil multiplicity.
-template <typename T, int DIM, bool MULT, typename BeadFn>
-__device__ __forceinline__ void pair_window_both(BeadFn bead, int m, const Prm<T> &P, int nbins, T &Apq, T &Aqp, T &C,
-                                                 bool &hit)
-{
-    const T ctau = T(-0.5) * P.tau;
-    T e0[4], u0[4]; // the previous slice's pair potential and multiplicity: oo, no, on, nn
-    bool in0[4];
-    Apq = Aqp = C = T(0);
-    hit = false;
-    for (int t = 0; t <= m; ++t) {
-        T po[DIM], pn[DIM], qo[DIM], qn[DIM];
-        bead(t, 0, po, pn);
-        bead(t, 1, qo, qn);
-        const T *x[4] = {po, pn, po, pn}, *y[4] = {qo, qo, qn, qn};
-        T e[4], u[4], tl[4];
-        bool in[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const T d2 = dist2_min<T, DIM>(x[k], y[k], P);
-            in[k] = d2 <= P.h2;
-            e[k] = vpair_r2(d2, P);
-            u[k] = MULT ? stencil_mult<T, DIM>(x[k], y[k], P, nbins) : T(1);
-        }
-        if (t > 0) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) tl[k] = in0[k] ? link_term<MULT>(u0[k], ctau, e0[k], e[k]) : T(0);
-            const T a1 = sub_(tl[1], tl[0]);
-            Apq = add_(Apq, a1);
-            Aqp = add_(Aqp, sub_(tl[2], tl[0]));
-            C = add_(C, sub_(sub_(tl[3], tl[2]), a1));
-        }
-        if (t < m) hit = hit || in[0] || in[1] || in[2] || in[3];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            e0[k] = e[k];
-            in0[k] = in[k];
-            if (MULT) u0[k] = u[k];
-        }
-    }
 }
 
 // Phase 1 of the centre-of-mass moves: one workgroup per (window, chain),
@@ -1035,11 +1149,11 @@ __global__ void __launch_bounds__(1024) k_com_spec(SweepArgs a, ComBuf<T> B, int
     const ComSpecLds L = com_spec_lds(N, lc, DIM, (int)sizeof(T), R, cap);
     T *const ob = reinterpret_cast<T *>(smem + L.ob), *const sd = reinterpret_cast<T *>(smem + L.sd);
     double *const sp = reinterpret_cast<double *>(smem + L.sp);
-    unsigned long long *const rmask = reinterpret_cast<unsigned long long *>(smem + L.rmask);
+    unsigned long long *const rmask = reinterpret_cast<unsigned long long *>(smem + L.pa);
     unsigned long long *const cmask = reinterpret_cast<unsigned long long *>(smem + L.cmask);
     int *const roff = reinterpret_cast<int *>(smem + L.roff), *const misc = reinterpret_cast<int *>(smem + L.misc);
     unsigned short *const coff = reinterpret_cast<unsigned short *>(smem + L.coff);
-    unsigned char *const prow = smem + L.prow;
+    unsigned short *const prow = reinterpret_cast<unsigned short *>(smem + L.prow);
     unsigned short *const pk = reinterpret_cast<unsigned short *>(smem + L.pk);
     unsigned short *const pq = reinterpret_cast<unsigned short *>(smem + L.pq);
     T *const pa_ = reinterpret_cast<T *>(smem + L.pa), *const pb_ = reinterpret_cast<T *>(smem + L.pb);
@@ -1120,7 +1234,7 @@ __global__ void __launch_bounds__(1024) k_com_spec(SweepArgs a, ComBuf<T> B, int
                 const unsigned long long bal = rmask[(size_t)l * nq + (k0 >> 6)];
                 if ((bal >> lane) & 1ull) {
                     const int s = at + __popcll(bal & ((1ull << lane) - 1ull)), q = row[k0 + lane];
-                    prow[s] = (unsigned char)l;
+                    prow[s] = (unsigned short)l;
                     pk[s] = (unsigned short)(k0 + lane);
                     pq[s] = (unsigned short)q;
                     atomicOr(cmask + (size_t)q * nc + (l >> 6), 1ull << (l & 63));
@@ -1299,7 +1413,8 @@ __global__ void __launch_bounds__(1024) k_com_dec(SweepArgs a, ComBuf<T> B, int 
         if (wave > 0) {
             fetch(chunk(k ^ 1), pa + nf, 1);
         } else {
-            const unsigned long long am = chunk_decide<T>(x.q, x.c, lane < nf ? x.off[lane] : 0, lane < nf ? x.off[lane + 1] : 0,
+            const unsigned long long am = chunk_decide<T>([&](int i) { return (int)x.q[i]; }, [&](int i) { return x.c[i]; },
+                                                          lane < nf ? x.off[lane] : 0, lane < nf ? x.off[lane + 1] : 0,
                                                           lane < nf ? s_spec[pa + lane] : 0.0, lane < nf ? su[pa + lane] : T(0),
                                                           pa, nf, acc);
             if (lane < nf) acc[pa + lane] = (unsigned char)((am >> lane) & 1ull);
