@@ -21,6 +21,7 @@ HEADERS = [
     "philox.hpp",
     "physics.hpp",
     "sweep_kernels.hpp",
+    "allpairs_kernels.hpp",
     "ideal_kernels.hpp",
     "hook_kernels.hpp",
     "window_kernels.hpp",
