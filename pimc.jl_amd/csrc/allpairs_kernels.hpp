@@ -392,4 +392,59 @@ template <typename T, int DIM> __global__ void __launch_bounds__(kAllPairsThread
     }
 }
 
+// Estimators of these chains in measuring runs that take them outside the sweep
+// kernel: grid (windows of kMeasSlices slices, chains of a.ids), 256 threads.  The
+// window's beads in LDS, one pair of particles per thread over the window's links
+// (each unordered pair once, with the weight of both ends); the single-bead terms
+// as measure_beads takes them.  part[(y * nblk + window) * 6]: the window's sums,
+// folded in window order by k_meas_fold.
+constexpr int kMeasSlices = 16;
+template <typename T, int DIM> __global__ void __launch_bounds__(256) k_meas_allpairs(MeasArgs a)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ double s_sum[6 * 16];
+    if (!split_measured(a)) return;
+    const int y = blockIdx.y, c = a.ids[y], tid = threadIdx.x, nt = blockDim.x;
+    ChainDev ch = a.chains[c];
+    const int N = ch.N, M = ch.M, s0 = blockIdx.x * kMeasSlices;
+    double *out = a.part + ((size_t)y * a.nblk + blockIdx.x) * 6;
+    if (s0 >= M) {
+        if (tid < 6) out[tid] = 0.0;
+        return;
+    }
+    const int m = min(kMeasSlices, M - s0);
+    const Prm<T> P = reinterpret_cast<const Prm<T> *>(a.prm)[c];
+    T *const gpath = reinterpret_cast<T *>(const_cast<void *>(a.pos)) + ch.pos_off;
+    T *const ob = reinterpret_cast<T *>(smem); // [slice][particle][d]
+    for (int i = tid; i < (m + 1) * N * DIM; i += nt) {
+        const int t = i / (N * DIM), j = s0 + t < M ? s0 + t : 0;
+        ob[i] = gpath[(size_t)j * N * DIM + (i - t * N * DIM)];
+    }
+    __syncthreads();
+    const double inv_s2 = 1.0 / (ch.sigma * ch.sigma), wq = 2.0 * (0.5 * (0.5 * (double)P.tau));
+    ch.pair = kPairNone; // the single-bead terms
+    const Path<T, DIM, true> path{gpath, M, N};
+    const Cells none{nullptr, nullptr, nullptr, M, 0, 0, ch.nbins};
+    ChainMeas r = measure_beads<T, DIM, false>(path, none, ch, P, a.radial, a.radial_bins, a.radial_winv, a.cart,
+                                               a.cart_bins, c, 1, nullptr, s0 * N, (s0 + m) * N);
+    // pairs q < p: thread i takes pairs i, i + nt, ... of the triangle, row by row
+    const int pairs = N * (N - 1) / 2;
+    int p = 1, q = tid;
+    for (int i = tid; i < pairs; i += nt, q += nt) {
+        while (q >= p) q -= p, ++p;
+        const T *rp = ob + (size_t)p * DIM, *rq = ob + (size_t)q * DIM;
+        pair_energy_window<T, DIM>([&](int t, T *x, T *z) {
+#pragma unroll
+            for (int e = 0; e < DIM; ++e) {
+                x[e] = rp[(size_t)t * N * DIM + e];
+                z[e] = rq[(size_t)t * N * DIM + e];
+            }
+        }, m, P, 3, wq, inv_s2, r.su, r.rgp);
+    }
+    double v[6] = {r.link, r.V, r.rg, r.su, r.rgp, r.r2w};
+    block_sums(v, s_sum);
+    if (tid == 0)
+        for (int k = 0; k < 6; ++k) out[k] = v[k];
+}
+
 } // namespace pimc

@@ -63,27 +63,6 @@ __host__ __device__ inline IdealLds ideal_lds(const ChainDev &h, int tsize)
     return ideal_lds(h.N, h.M, h.dim, tsize, h.swaps, h.swap_m);
 }
 
-// NV workgroup sums at once (block_sum's order each); buf: NV x 16 doubles.
-template <int NV> __device__ inline void block_sums(double (&v)[NV], double *buf)
-{
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1)
-#pragma unroll
-        for (int k = 0; k < NV; ++k) v[k] += __shfl_xor(v[k], off, 64);
-    if (lane == 0)
-#pragma unroll
-        for (int k = 0; k < NV; ++k) buf[k * 16 + wave] = v[k];
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-        double s = 0.0;
-        for (int w = 0; w < nw; ++w) s += buf[k * 16 + w];
-        v[k] = s;
-    }
-    __syncthreads();
-}
-
 template <typename T, int DIM> __global__ void __launch_bounds__(kIdealThreads) k_sweep_ideal(SweepArgs a)
 {
     extern __shared__ __align__(16) unsigned char smem[];

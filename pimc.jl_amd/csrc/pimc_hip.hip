@@ -113,7 +113,9 @@ struct pimc_ctx {
     size_t lds_ideal = 0;
     std::vector<int> allpairs_ids;     // small Gaussian-pair chains, on k_sweep_allpairs
     int *d_allpairs = nullptr, allpairs_g = 2;
-    size_t lds_allpairs = 0;
+    size_t lds_allpairs = 0, lds_apmeas = 0;
+    int apmeas_nblk = 1;
+    double *d_apmeas_part = nullptr;   // their split estimators' partial sums [id][window][6]
     // Gaussian-pair chains on the window staging and centre-of-mass kernels, with and without
     // cell lists for the estimators (index 0: cells, 1: all-pairs); win_all: both
     std::vector<int> win_ids[2], win_all;
@@ -616,6 +618,20 @@ template <typename T, int DIM> void launch_meas_d(pimc_ctx *c, int sweep_off)
         m.n_ids = nall;
         m.part = c->d_meas_part;
         hipLaunchKernelGGL(k_meas_fold, dim3((unsigned)((nall + 127) / 128)), dim3(128), 0, c->stream, m);
+        HIPCHK(hipGetLastError());
+    }
+    const int nap = c->split_meas ? (int)c->allpairs_ids.size() : 0;
+    if (nap > 0) {
+        m.ids = c->d_allpairs;
+        m.n_ids = nap;
+        m.nblk = c->apmeas_nblk;
+        m.part = c->d_apmeas_part;
+        auto k = k_meas_allpairs<T, DIM>;
+        if (c->lds_apmeas > 65536) HIPCHK(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->lds_apmeas));
+        hipLaunchKernelGGL(k, dim3((unsigned)c->apmeas_nblk, (unsigned)nap), dim3(256),
+                           c->lds_apmeas, c->stream, m);
+        HIPCHK(hipGetLastError());
+        hipLaunchKernelGGL(k_meas_fold, dim3((unsigned)((nap + 127) / 128)), dim3(128), 0, c->stream, m);
         HIPCHK(hipGetLastError());
     }
 }
@@ -1429,6 +1445,8 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
             for (int id : c->allpairs_ids) {
                 const ChainDev &h = c->ch[id];
                 c->lds_allpairs = std::max(c->lds_allpairs, allpairs_lds(h.N, h.M, h.dim, ts, c->allpairs_g).end);
+                c->lds_apmeas = std::max(c->lds_apmeas, (size_t)(std::min(kMeasSlices, h.M) + 1) * h.N * h.dim * ts);
+                c->apmeas_nblk = std::max(c->apmeas_nblk, (h.M + kMeasSlices - 1) / kMeasSlices);
             }
         }
         // tabulated-propagator chains last in each list (their own kernel instantiation)
@@ -1468,7 +1486,6 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
                 c->meas_ids.insert(c->meas_ids.end(), c->whole_brute_ids.begin(), c->whole_brute_ids.end());
                 c->meas_ids.insert(c->meas_ids.end(), c->whole_lds_ids.begin(), c->whole_lds_ids.end());
                 c->meas_ids.insert(c->meas_ids.end(), c->ideal_ids.begin(), c->ideal_ids.end());
-                c->meas_ids.insert(c->meas_ids.end(), c->allpairs_ids.begin(), c->allpairs_ids.end());
             }
             long long most = 0;
             for (int id : c->meas_ids) most = std::max(most, (long long)c->ch[id].N * c->ch[id].M);
@@ -1527,6 +1544,7 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
         c->d_whole_brute = dalloc<int>(c->whole_brute_ids.size());
         c->d_whole_lds = dalloc<int>(c->whole_lds_ids.size());
         c->d_allpairs = dalloc<int>(c->allpairs_ids.size());
+        c->d_apmeas_part = dalloc<double>(c->allpairs_ids.size() * (size_t)c->apmeas_nblk * 6);
         if (!c->allpairs_ids.empty())
             HIPCHK(hipMemcpy(c->d_allpairs, c->allpairs_ids.data(), sizeof(int) * c->allpairs_ids.size(), hipMemcpyHostToDevice));
         c->d_ideal = dalloc<int>(c->ideal_ids.size());
@@ -1720,7 +1738,7 @@ int pimc_destroy(pimc_ctx *c)
                     c->d_whole_cells, c->d_whole_brute, c->d_is_whole, c->d_cell_cnt, c->d_bins, c->d_cell_mem,
                     c->d_status, c->d_work, c->d_io, c->d_whole_lds, c->d_next, c->d_meas_ids, c->d_meas_part,
                     c->d_cells_all, c->d_spec, c->d_wbnd, c->d_win_all, c->d_cacc, c->d_cshift, c->d_rbnd, c->d_ccnt, c->d_partner, c->d_cval, c->d_win_part,
-                    c->d_beams, c->d_wg_cells[0], c->d_wg_cells[1], c->d_hpart, c->d_dens, c->d_ideal, c->d_allpairs};
+                    c->d_beams, c->d_wg_cells[0], c->d_wg_cells[1], c->d_hpart, c->d_dens, c->d_ideal, c->d_allpairs, c->d_apmeas_part};
     for (void *p : ptrs) dfree(p);
     for (double *p : c->d_tab) dfree(p);
     if (c->h_pin) (void)hipHostFree(c->h_pin);

@@ -874,6 +874,26 @@ __device__ inline double block_sum(double v, double *wbuf)
     return s;
 }
 
+// NV workgroup sums at once (block_sum's order each); buf: NV x 16 doubles.
+template <int NV> __device__ inline void block_sums(double (&v)[NV], double *buf)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < NV; ++k) v[k] += __shfl_xor(v[k], off, 64);
+    if (lane == 0)
+#pragma unroll
+        for (int k = 0; k < NV; ++k) buf[k * 16 + wave] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        double s = 0.0;
+        for (int w = 0; w < nw; ++w) s += buf[k * 16 + w];
+        v[k] = s;
+    }
+    __syncthreads();
+}
 
 // Squared periodic distance of two beads.
 template <typename T, int DIM> __device__ __forceinline__ T dist2(const T *x, const T *y, const Prm<T> &P)

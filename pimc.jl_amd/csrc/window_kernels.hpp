@@ -1473,6 +1473,33 @@ __host__ __device__ inline MeasWinLds meas_win_lds(int N, int lc, int dim, int t
     return L;
 }
 
+// Pair energy and pair virial of one pair over the slices 0 .. m - 1 of a window,
+// added to su and rg with weight wq per link and stencil multiplicity: the terms of
+// pair_energy_bead.  Each bead pair's distance and exponential serve the link
+// before it and the link after it.  bead(t, x, y): the pair's beads at slice t.
+template <typename T, int DIM, typename BeadFn>
+__device__ __forceinline__ void pair_energy_window(BeadFn bead, int m, const Prm<T> &P, int nbins, double wq, double inv_s2,
+                                                   double &su, double &rg)
+{
+    T x[DIM], y[DIM];
+    bead(0, x, y);
+    T r2 = dist2_min<T, DIM>(y, x, P);
+    double ea = (double)ex(-r2 * P.inv2s2);
+    for (int t = 0; t < m; ++t) {
+        const bool in = r2 <= P.h2;
+        const double wt = nbins >= 3 ? wq : wq * (double)stencil_mult<T, DIM>(x, y, P, nbins);
+        bead(t + 1, x, y);
+        const T s2 = dist2_min<T, DIM>(y, x, P);
+        const double eb = (double)ex(-s2 * P.inv2s2);
+        if (in) {
+            su += wt * (ea + eb);
+            rg += wt * (-((double)r2 * inv_s2) * ea - ((double)s2 * inv_s2) * eb);
+        }
+        r2 = s2;
+        ea = eb;
+    }
+}
+
 // Estimators of Gaussian-pair chains after a sweep, by the centre-of-mass
 // windows: one 512-thread workgroup per (window, chain of a.ids).  The terms of
 // measure_chain for the beads of slices s0 .. s0 + m - 1: kinetic link to the
@@ -1593,17 +1620,14 @@ template <typename T, int DIM> __global__ void __launch_bounds__(512) k_meas_win
         const int total = X.misc[1];
         for (int i = tid; i < total; i += nt) {
             const int p = pa + X.po[i], q = X.pq[i];
-            for (int t = 0; t < m; ++t) {
-                const T *rp = ob + ((size_t)t * N + p) * DIM, *rq = ob + ((size_t)t * N + q) * DIM;
-                const T r2 = dist2<T, DIM>(rq, rp, P);
-                if (!(r2 <= P.h2)) continue;
-                const T mult = stencil_mult<T, DIM>(rp, rq, P, ch.nbins);
-                const T s2 = dist2<T, DIM>(rq + (size_t)N * DIM, rp + (size_t)N * DIM, P);
-                const double ea = (double)ex(-r2 * P.inv2s2), eb = (double)ex(-s2 * P.inv2s2);
-                const double wt = wq * (double)mult;
-                su += wt * (ea + eb);
-                rgp += wt * (-((double)r2 * inv_s2) * ea - ((double)s2 * inv_s2) * eb);
-            }
+            const T *rp = ob + (size_t)p * DIM, *rq = ob + (size_t)q * DIM;
+            pair_energy_window<T, DIM>([&](int t, T *x, T *y) {
+#pragma unroll
+                for (int e = 0; e < DIM; ++e) {
+                    x[e] = rp[(size_t)t * N * DIM + e];
+                    y[e] = rq[(size_t)t * N * DIM + e];
+                }
+            }, m, P, ch.nbins, wq, inv_s2, su, rgp);
         }
         __syncthreads();
         pa += nf;
