@@ -655,7 +655,10 @@ template <typename T> struct StagePairs {
 // is evaluated once, for A(p, q), A(q, p) and C(p, q), one pair per thread.  When
 // every pair is done the tries are decided chunk by chunk.  Pair terms are VALU
 // work (four pairings a slice); two workgroups share a CU, so one's decisions,
-// a serial chain, run beside the other's pairs.
+// a serial chain, run beside the other's pairs.  Against pair slots per chunk of 64
+// tries, each pair from both sides (six pairings): 16 measuring sweeps of 256 chains
+// of N = 256, M = 128, FP32, 45.2 -> 40.0 ms; 64 chains of N = 400, M = 512, whose
+// blocks fill a CU alone, stay at 65 to 67 ms.
 template <typename T, int DIM>
 __global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, int R, int cap, int keep, int budget)
 {
@@ -1129,7 +1132,8 @@ __host__ __device__ inline ComSpecLds com_spec_lds(int N, int lc, int dim, int t
 // window bounds, evaluated one per thread, and each particle's sum takes its
 // partners by index (the block's own rows first, then the rows that name it).
 // The pair terms are VALU work, four pairings of two beads a slice; a pool of the
-// whole window's pairs keeps the threads evenly loaded.
+// whole window's pairs keeps the threads evenly loaded.  All C here instead of those
+// of accepted partners in k_com_dec: more pairs, but on every CU (see k_com_dec).
 template <typename T, int DIM>
 __global__ void __launch_bounds__(1024) k_com_spec(SweepArgs a, ComBuf<T> B, int R, int cap)
 {
@@ -1324,7 +1328,10 @@ __host__ __device__ inline ComDecLds com_dec_lds(int N, int tsize, int cap)
 // tries the listed pairs' C values are added over the windows (window order; zero
 // outside reach) into LDS, and one wave decides the chunk in rounds while the
 // other waves fetch the next chunk's.  What bounds it is the serial chain of
-// rounds of that wave.  cacc[part]: 1 when the particle's try was accepted.
+// rounds of that wave.  With 64 chains (N = 400, M = 512, FP32) on 64 of 256 CUs it
+// took 1.78 ms a sweep while it evaluated the C terms itself, 0.21 ms now; 16
+// measuring sweeps 77.5 -> 65.0 ms, and 49.3 -> 45.2 ms for 256 chains of N = 256,
+// M = 128.  cacc[part]: 1 when the particle's try was accepted.
 template <typename T, int DIM>
 __global__ void __launch_bounds__(1024) k_com_dec(SweepArgs a, ComBuf<T> B, int cap, unsigned char *cacc)
 {
@@ -1476,7 +1483,9 @@ __host__ __device__ inline MeasWinLds meas_win_lds(int N, int lc, int dim, int t
 // Pair energy and pair virial of one pair over the slices 0 .. m - 1 of a window,
 // added to su and rg with weight wq per link and stencil multiplicity: the terms of
 // pair_energy_bead.  Each bead pair's distance and exponential serve the link
-// before it and the link after it.  bead(t, x, y): the pair's beads at slice t.
+// before it and the link after it (16 measuring sweeps of 256 chains of N = 256,
+// M = 128, FP32: 40.0 ms with two exponentials per link, 39.4 ms with one per slice).
+// bead(t, x, y): the pair's beads at slice t.
 template <typename T, int DIM, typename BeadFn>
 __device__ __forceinline__ void pair_energy_window(BeadFn bead, int m, const Prm<T> &P, int nbins, double wq, double inv_s2,
                                                    double &su, double &rg)
