@@ -338,8 +338,8 @@ template <int DIM, typename Visit> __device__ __forceinline__ void grid_visit(co
 
 // Slots of the chunk's particles pa, pa + 1, ... (at most kc <= kChunk): for
 // each the partners q with cand(p, q), by index.  Fills as many particles as
-// the pool holds (at least one: cap >= N).  Returns the number of particles filled; X.misc[1] is the
-// slot count.  All threads of the workgroup.
+// the pool holds (at least one: cap >= N).  Returns the number of particles filled (0: a caller's
+// loop over the particles has to end); X.misc[1] is the slot count.  All threads of the workgroup.
 template <int DIM = 2, typename T, typename Cand>
 __device__ inline int chunk_slots(ChunkPtr<T> &X, int pa, int N, int cap, int kc, Cand cand,
                                   const WinGrid *G = nullptr)
@@ -385,10 +385,11 @@ __device__ inline int chunk_slots(ChunkPtr<T> &X, int pa, int N, int cap, int kc
         const bool fits = lane < nc && pre + v <= cap;
         const int nf = __popcll(__ballot(fits));
         X.off[lane] = pre;
-        if (lane == nf - 1) {
+        if (lane == 0) {
             X.misc[0] = nf;
-            X.misc[1] = pre + v;
+            X.misc[1] = 0; // none filled: no slots
         }
+        if (lane == nf - 1) X.misc[1] = pre + v;
     }
     __syncthreads();
     const int nf = X.misc[0];
@@ -419,10 +420,12 @@ __device__ inline int chunk_slots(ChunkPtr<T> &X, int pa, int N, int cap, int kc
 // round decides every try whose such partners are decided; a try's sum takes the
 // partners before the chunk in index order, then the partners inside the chunk as
 // they are accepted (by round, in index order within a round), a fixed order.
+// The earliest undecided try is always ready, so nf rounds decide the chunk; a list that names a
+// partner at or after its own try would leave tries undecided (not accepted), and `whole` is false.
 // Returns the acceptance mask.
 template <typename T, typename Q, typename C>
 __device__ inline unsigned long long chunk_decide(Q pq, C pc, int o0, int o1, double sp, T u, int pa, int nf,
-                                                  const unsigned char *acc)
+                                                  const unsigned char *acc, bool &whole)
 {
     const int l = threadIdx.x & 63;
     const bool in = l < nf;
@@ -440,7 +443,7 @@ __device__ inline unsigned long long chunk_decide(Q pq, C pc, int o0, int o1, do
         }
     }
     unsigned long long decided = nf >= 64 ? 0ull : (~0ull << nf), am = 0ull;
-    while (decided != ~0ull) {
+    for (int round = 0; round < nf && decided != ~0ull; ++round) {
         const bool ready = in && !((decided >> l) & 1ull) && (dep & ~decided) == 0ull;
         bool ok = false;
         if (ready) {
@@ -459,6 +462,7 @@ __device__ inline unsigned long long chunk_decide(Q pq, C pc, int o0, int o1, do
             }
         }
     }
+    whole = decided == ~0ull;
     return am;
 }
 
@@ -856,6 +860,10 @@ __global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, in
         }
         __syncthreads();
         const int nf = misc[0], total = poff[pa + nf] - base;
+        if (nf < 1) { // uniform; not reached while a row's pairs fit the pool (cap >= N)
+            if (tid == 0) atomicOr(a.status + c, 2);
+            return;
+        }
         for (int it = tid; it < nf * nq; it += nt) {
             const int l = it / nq, wd = it - l * nq;
             if (wd * 64 >= pa + l) continue;
@@ -923,11 +931,17 @@ __global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, in
             int tot;
             const int pre = wave_prefix(v, lane, tot);
             const int nf = __popcll(__ballot(p < N && pre + v <= budget));
+            if (nf < 1) { // not reached while a try's partners fit (budget >= N)
+                if (lane == 0) atomicOr(a.status + c, 2);
+                break;
+            }
+            bool whole;
             const bool in = lane < nf;
             const T u = Uniform<T>::get(draw(a.seed, (uint32_t)(p * M + s0), sw, (uint32_t)c, kLevyAccept).x);
             const unsigned long long am = chunk_decide<T>([&](int i) { return S.q(i); }, [&](int i) { return S.c(i); },
                                                           in ? poff[p] : 0, in ? poff[p + 1] : 0, in ? sp[p] : 0.0, u,
-                                                          pa, nf, acc);
+                                                          pa, nf, acc, whole);
+            if (!whole && lane == 0) atomicOr(a.status + c, 2);
             if (in) acc[p] = (unsigned char)((am >> lane) & 1ull);
             __builtin_amdgcn_wave_barrier(); // the next chunk reads the decisions
             lacc += __popcll(am);
@@ -1230,6 +1244,10 @@ __global__ void __launch_bounds__(1024) k_com_spec(SweepArgs a, ComBuf<T> B, int
         }
         __syncthreads();
         const int nf = misc[0], total = roff[nf];
+        if (nf < 1) { // uniform; not reached while a row's pairs fit the pool (cap >= N)
+            if (tid == 0) atomicOr(a.status + c, 2);
+            return;
+        }
         for (int l = wave; l < nf; l += nwv) {
             const int p = pa + l, n = B.cnt[part + p];
             const unsigned short *row = B.row(ch, p);
@@ -1378,10 +1396,8 @@ __global__ void __launch_bounds__(1024) k_com_dec(SweepArgs a, ComBuf<T> B, int 
         const int nf = __popcll(__ballot(pa + lane < N && pre + v <= cap));
         if (wave == w0) {
             x.off[lane] = pre;
-            if (lane == nf - 1) {
-                x.off[nf] = pre + v;
-                *x.n = nf;
-            }
+            if (lane == nf - 1) x.off[nf] = pre + v;
+            if (lane == 0) *x.n = nf;
         }
         for (int l = wave - w0; l < nf; l += nwv - w0) {
             const int p = pa + l, n = __shfl(v, l, 64), o = __shfl(pre, l, 64);
@@ -1417,13 +1433,19 @@ __global__ void __launch_bounds__(1024) k_com_dec(SweepArgs a, ComBuf<T> B, int 
     for (int pa = 0, k = 0; pa < N; k ^= 1) {
         const Chunk x = chunk(k);
         const int nf = *x.n;
+        if (nf < 1) { // uniform; not reached while a try's partners fit (cap >= N)
+            if (tid == 0) atomicOr(a.status + c, 2);
+            break;
+        }
         if (wave > 0) {
             fetch(chunk(k ^ 1), pa + nf, 1);
         } else {
+            bool whole;
             const unsigned long long am = chunk_decide<T>([&](int i) { return (int)x.q[i]; }, [&](int i) { return x.c[i]; },
                                                           lane < nf ? x.off[lane] : 0, lane < nf ? x.off[lane + 1] : 0,
                                                           lane < nf ? s_spec[pa + lane] : 0.0, lane < nf ? su[pa + lane] : T(0),
-                                                          pa, nf, acc);
+                                                          pa, nf, acc, whole);
+            if (!whole && lane == 0) atomicOr(a.status + c, 2);
             if (lane < nf) acc[pa + lane] = (unsigned char)((am >> lane) & 1ull);
             nacc += __popcll(am);
         }
@@ -1626,6 +1648,7 @@ template <typename T, int DIM> __global__ void __launch_bounds__(512) k_meas_win
             const float4 A = bnd[p], B = bnd[q];
             return bnd_near<DIM>(A.x, A.y, A.z, B.x, B.y, B.z, h, twoL, inv2L);
         }, &G);
+        if (nf < 1) break; // uniform; not reached (cap >= N)
         const int total = X.misc[1];
         for (int i = tid; i < total; i += nt) {
             const int p = pa + X.po[i], q = X.pq[i];
