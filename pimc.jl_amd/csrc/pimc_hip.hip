@@ -1337,9 +1337,7 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
                 if (win) {
                     const int N = std::max(c->win_maxN, h.N), ell = std::max(c->win_maxell, h.ell);
                     const int lc = std::max(com_win_len(std::max(c->win_maxM, h.M)), 8);
-                    win = stage_lds(N, ell, h.dim, tsz, 64, N, 0).end <= 160 * 1024 &&
-                          com_spec_lds(N, lc, h.dim, tsz, 64, N).end <= 160 * 1024 &&
-                          com_dec_lds(N, tsz, N).end <= 160 * 1024;
+                    win = win_fits(N, ell, lc, h.dim, tsz);
                 }
                 if (cells) {
                     h.ncell = (int)ncell;

@@ -1502,6 +1502,17 @@ __host__ __device__ inline MeasWinLds meas_win_lds(int N, int lc, int dim, int t
     return L;
 }
 
+// Whether the LDS of a workgroup holds the smallest blocks and pools of all four kernels that a
+// window chain runs on (N, ell and lc the largest of the chains that share their launches): 160 KiB,
+// of which k_meas_win has kMeasWinStatic in arrays of its own.
+constexpr size_t kMeasWinStatic = 32 * sizeof(double);
+inline bool win_fits(int N, int ell, int lc, int dim, int tsize)
+{
+    const size_t most = 160 * 1024;
+    return stage_lds(N, ell, dim, tsize, 64, N, 0).end <= most && com_spec_lds(N, lc, dim, tsize, 64, N).end <= most &&
+           com_dec_lds(N, tsize, N).end <= most && meas_win_lds(N, lc, dim, tsize, N).ck.end + kMeasWinStatic <= most;
+}
+
 // Pair energy and pair virial of one pair over the slices 0 .. m - 1 of a window,
 // added to su and rg with weight wq per link and stencil multiplicity: the terms of
 // pair_energy_bead.  Each bead pair's distance and exponential serve the link
@@ -1543,7 +1554,7 @@ __device__ __forceinline__ void pair_energy_window(BeadFn bead, int m, const Prm
 template <typename T, int DIM> __global__ void __launch_bounds__(512) k_meas_win(MeasArgs a, int nwin, int cap)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ double wbuf[32];
+    __shared__ double wbuf[kMeasWinStatic / sizeof(double)];
     if (!split_measured(a)) return;
     const int y = blockIdx.y, c = a.ids[y], w = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
     const ChainDev ch = a.chains[c];
