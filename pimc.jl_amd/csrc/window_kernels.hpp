@@ -384,12 +384,12 @@ __device__ inline int chunk_slots(ChunkPtr<T> &X, int pa, int N, int cap, int kc
         const int pre = wave_prefix(v, lane, tot);
         const bool fits = lane < nc && pre + v <= cap;
         const int nf = __popcll(__ballot(fits));
+        const int used = __shfl(pre + v, max(nf - 1, 0), 64);
         X.off[lane] = pre;
         if (lane == 0) {
             X.misc[0] = nf;
-            X.misc[1] = 0; // none filled: no slots
+            X.misc[1] = nf > 0 ? used : 0;
         }
-        if (lane == nf - 1) X.misc[1] = pre + v;
     }
     __syncthreads();
     const int nf = X.misc[0];
