@@ -593,13 +593,18 @@ inline int stage_budget(int N, int ell, int dim, int tsize)
 }
 
 // LDS of k_stage_win: old beads of the window's ell + 1 slices, new interior
-// beads, bounds, sums, decisions, grid; masks of a block of R rows
+// beads, bounds, sums, candidate counts, grid; masks of a block of R rows
 // (partners q < p in words of 64, and each particle's rows), the block's pool of
-// cap pairs (row and the two A values), then the window's pairs by row: partner
+// cap pairs (the two A values), then the window's pairs by row: partner
 // with the hit flag in bit 15 and C, the first `keep` of them here and the rest
-// in memory.
+// in memory.  What one workgroup needs with the smallest blocks (R = 64, cap = N,
+// keep = 0) sets the largest chain, so arrays that are not in use together share
+// their place: the A values follow the row masks, the decisions the column masks,
+// a row's end in the pair list is the fourth word of its particle's bound, and a
+// pair's row waits in the place of its C.  2D FP32, ell = 8: N <= 922; 868 with a
+// place each.
 struct StageLds {
-    size_t ob, nb, bnd, sp, acc, ncand, off, cmask, coff, misc, prow, pa, pb, pq, pc, end;
+    size_t ob, nb, bnd, sp, ncand, cmask, coff, misc, pa, pq, pc, end;
     GridLds gr;
 };
 __host__ __device__ inline StageLds stage_lds(int N, int ell, int dim, int tsize, int R, int cap, int keep)
@@ -615,18 +620,14 @@ __host__ __device__ inline StageLds stage_lds(int N, int ell, int dim, int tsize
     L.nb = take((size_t)(ell > 1 ? ell - 1 : 1) * N * dim * tsize);
     L.bnd = take((size_t)N * 16);
     L.sp = take((size_t)N * 8);
-    L.acc = take((size_t)N);
     L.ncand = take((size_t)N * 2);
-    L.off = take((size_t)(N + 1) * 4);
     L.gr = grid_lds(o, N, dim);
     o = L.gr.end;
-    L.cmask = take((size_t)N * (R / 64) * 8);
+    L.cmask = take((size_t)N * (R / 64) * 8); // after the last block: the decisions
     L.coff = take((size_t)N * 2);
     L.misc = take(16);
-    L.prow = take((size_t)cap * 2);
-    const size_t rows = (size_t)R * ((N + 63) / 64) * 8, vals = (size_t)cap * tsize;
-    L.pa = take(rows > vals ? rows : vals); // the row masks, then the A(p, q)
-    L.pb = take(vals);
+    const size_t rows = (size_t)R * ((N + 63) / 64) * 8, vals = 2 * (size_t)cap * tsize;
+    L.pa = take(rows > vals ? rows : vals); // the row masks, then the A(p, q) and the A(q, p)
     L.pq = take((size_t)keep * 2);
     L.pc = take((size_t)keep * tsize);
     L.end = o;
@@ -648,6 +649,19 @@ template <typename T> struct StagePairs {
             gq[i] = (unsigned short)q;
             gc[i] = c;
         }
+    }
+    // before it is evaluated, pair i's row in the place of its C
+    __device__ __forceinline__ void put_row(int i, int q, int l) const
+    {
+        T c;
+        if constexpr (sizeof(T) == 4) c = __int_as_float(l);
+        else c = __longlong_as_double(l);
+        put(i, q, c);
+    }
+    __device__ __forceinline__ int row(int i) const
+    {
+        if constexpr (sizeof(T) == 4) return __float_as_int(c(i));
+        else return (int)__double_as_longlong(c(i));
     }
     __device__ __forceinline__ int q(int i) const { return i < keep ? lq[i] : gq[i]; }
     __device__ __forceinline__ T c(int i) const { return i < keep ? lc[i] : gc[i]; }
@@ -692,15 +706,17 @@ __global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, in
     T *nb = reinterpret_cast<T *>(smem + L.nb); // [t - 1][k][d], t = 1..m-1
     float4 *bnd = reinterpret_cast<float4 *>(smem + L.bnd);
     double *const sp = reinterpret_cast<double *>(smem + L.sp);
-    unsigned char *acc = smem + L.acc;
+    unsigned char *const acc = smem + L.cmask;
     unsigned short *const ncand = reinterpret_cast<unsigned short *>(smem + L.ncand);
-    int *const poff = reinterpret_cast<int *>(smem + L.off);
+    // row p's pairs are row_start(p) .. row_end(p) of the list
+    int *const bnd_w = reinterpret_cast<int *>(smem + L.bnd) + 3;
+    auto row_end = [&](int p) -> int & { return bnd_w[4 * p]; };
+    auto row_start = [&](int p) { return p > 0 ? bnd_w[4 * p - 4] : 0; };
     unsigned long long *const rmask = reinterpret_cast<unsigned long long *>(smem + L.pa);
     unsigned long long *const cmask = reinterpret_cast<unsigned long long *>(smem + L.cmask);
     unsigned short *const coff = reinterpret_cast<unsigned short *>(smem + L.coff);
     int *const misc = reinterpret_cast<int *>(smem + L.misc);
-    unsigned short *const prow = reinterpret_cast<unsigned short *>(smem + L.prow);
-    T *const pa_ = reinterpret_cast<T *>(smem + L.pa), *const pb_ = reinterpret_cast<T *>(smem + L.pb);
+    T *const pa_ = reinterpret_cast<T *>(smem + L.pa), *const pb_ = pa_ + cap;
     const size_t tri = pair_row(N);
     T *const gval = B.vals(ch, 0);
     const StagePairs<T> S{reinterpret_cast<T *>(smem + L.pc), gval + (size_t)w * tri,
@@ -778,10 +794,8 @@ __global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, in
         }
         bnd[p] = make_float4(ref[0] + mean[0], DIM > 1 ? ref[DIM - 1] + mean[DIM - 1] : 0.f, sqrtf(r2), 0.f);
         sp[p] = (double)dv;
-        acc[p] = 0;
         ncand[p] = 0;
     }
-    if (tid == 0) poff[0] = 0;
     __syncthreads();
 
     const float h = (float)ch.h, twoL = (float)(2.0 * ch.L), inv2L = 1.0f / twoL;
@@ -810,7 +824,7 @@ __global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, in
     };
     const int nq = (N + 63) / 64, nc = R / 64; // words of a row mask, of a column mask
     for (int pa = 0; pa < N;) {
-        const int nr = min(R, N - pa), base = poff[pa];
+        const int nr = min(R, N - pa), base = row_start(pa);
         for (int i = tid; i < N * nc; i += nt) cmask[i] = 0ull;
         // partners q < p in reach of each row
         if (G.ng > 0) {
@@ -826,7 +840,7 @@ __global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, in
             for (int l = tid; l < nr; l += nt) {
                 int cnt = 0;
                 for (int k = 0; k < nq; ++k) cnt += __popcll(rmask[(size_t)l * nq + k]);
-                poff[pa + l + 1] = cnt;
+                row_end(pa + l) = cnt;
             }
         } else {
             for (int l = wave; l < nr; l += nwv) {
@@ -838,19 +852,19 @@ __global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, in
                     if (lane == 0) rmask[(size_t)l * nq + (q0 >> 6)] = bal;
                     cnt += __popcll(bal);
                 }
-                if (lane == 0) poff[p + 1] = cnt;
+                if (lane == 0) row_end(p) = cnt;
             }
         }
         __syncthreads();
         if (wave == 0) { // prefix; the rows whose pairs fit the pool
             int sum = 0, nf = 0;
             for (int l0 = 0; l0 < nr; l0 += 64) {
-                const int l = l0 + lane, v = l < nr ? poff[pa + l + 1] : 0;
+                const int l = l0 + lane, v = l < nr ? row_end(pa + l) : 0;
                 int tot;
                 const int pre = wave_prefix(v, lane, tot);
                 const bool fits = l < nr && sum + pre + v <= cap;
                 if (fits) {
-                    poff[pa + l + 1] = base + sum + pre + v;
+                    row_end(pa + l) = base + sum + pre + v;
                     ncand[pa + l] = (unsigned short)(ncand[pa + l] + v);
                 }
                 nf += __popcll(__ballot(fits));
@@ -859,23 +873,23 @@ __global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, in
             if (lane == 0) misc[0] = nf;
         }
         __syncthreads();
-        const int nf = misc[0], total = poff[pa + nf] - base;
+        const int nf = misc[0];
         if (nf < 1) { // uniform; not reached while a row's pairs fit the pool (cap >= N)
             if (tid == 0) atomicOr(a.status + c, 2);
             return;
         }
+        const int total = row_end(pa + nf - 1) - base;
         for (int it = tid; it < nf * nq; it += nt) {
             const int l = it / nq, wd = it - l * nq;
             if (wd * 64 >= pa + l) continue;
             const unsigned long long *mk = rmask + (size_t)l * nq;
-            int s = poff[pa + l] - base;
+            int s = row_start(pa + l) - base;
             for (int k = 0; k < wd; ++k) s += __popcll(mk[k]);
             unsigned long long b = mk[wd];
             while (b) {
                 const int q = wd * 64 + __ffsll((long long)b) - 1;
                 b &= b - 1;
-                prow[s] = (unsigned short)l;
-                S.put(base + s, q, T(0));
+                S.put_row(base + s, q, l);
                 atomicOr(cmask + (size_t)q * nc + (l >> 6), 1ull << (l & 63));
                 ++s;
             }
@@ -898,7 +912,7 @@ __global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, in
         }
         __syncthreads();
         for (int i = tid; i < total; i += nt) {
-            const int l = prow[i], p = pa + l, q = S.q(base + i);
+            const int l = S.row(base + i), p = pa + l, q = S.q(base + i);
             T Apq, Aqp, C;
             bool hit;
             if (ch.nbins >= 3) pair_window_both<T, DIM, false, true>(bead(p, q), m, P, ch.nbins, Apq, Aqp, C, hit);
@@ -914,7 +928,7 @@ __global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, in
         for (int x = tid; x < N; x += nt) { // partners by index: the particle's own row, then the rows that name it
             double s = sp[x];
             if (x >= pa && x < pa + nf)
-                for (int i = poff[x] - base; i < poff[x + 1] - base; ++i) s += (double)pa_[i];
+                for (int i = row_start(x) - base; i < row_end(x) - base; ++i) s += (double)pa_[i];
             int n = 0;
             for (int k = 0; k < nc; ++k) n += __popcll(cmask[(size_t)x * nc + k]);
             for (int i = coff[x]; i < coff[x] + n; ++i) s += (double)pb_[i];
@@ -933,13 +947,14 @@ __global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, in
             const int nf = __popcll(__ballot(p < N && pre + v <= budget));
             if (nf < 1) { // not reached while a try's partners fit (budget >= N)
                 if (lane == 0) atomicOr(a.status + c, 2);
+                for (int k = p; k < N; k += 64) acc[k] = 0;
                 break;
             }
             bool whole;
             const bool in = lane < nf;
             const T u = Uniform<T>::get(draw(a.seed, (uint32_t)(p * M + s0), sw, (uint32_t)c, kLevyAccept).x);
             const unsigned long long am = chunk_decide<T>([&](int i) { return S.q(i); }, [&](int i) { return S.c(i); },
-                                                          in ? poff[p] : 0, in ? poff[p + 1] : 0, in ? sp[p] : 0.0, u,
+                                                          in ? row_start(p) : 0, in ? row_end(p) : 0, in ? sp[p] : 0.0, u,
                                                           pa, nf, acc, whole);
             if (!whole && lane == 0) atomicOr(a.status + c, 2);
             if (in) acc[p] = (unsigned char)((am >> lane) & 1ull);

@@ -5,6 +5,7 @@ import pytest
 from pimc import _capi as A
 from pimc.potentials import GaussianPair, NoPotential
 from pimc.system import chain_desc
+from test_gpu_random_configs import run_and_check
 
 pytestmark = pytest.mark.gpu
 
@@ -36,3 +37,11 @@ def test_long_rings_are_measured_fp32(N, M):
     E, Ev, Ep, Evp = ctx.energy(0)
     assert abs(e.E - e.Epair - E) < 1e-6 * d.dim * N * M / d.beta
     assert abs(e.Epair - Ep) < 1e-6 * abs(Ep)
+
+
+@pytest.mark.parametrize("N,M,ell,L,nbins,dim", [(148, 40, 32, 4.0, 4, 2), (504, 9, 8, 8.0, 8, 2), (281, 36, 32, 60.0, 40, 1)])
+def test_largest_chains_match_oracle_fp64(N, M, ell, L, nbins, dim):
+    """The largest chains of their staging length: the smallest blocks, a pool of
+    one particle's partners, and nearly all pairs of a window in memory."""
+    d, r = gas(N, M, ell, L, nbins, dim)
+    run_and_check([(d, r, "gauss", (1, 1, 1))], 61 + N, 1)
