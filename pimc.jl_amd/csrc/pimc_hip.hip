@@ -647,8 +647,9 @@ void launch_meas(pimc_ctx *c, int sweep_off)
     }
 }
 
-// Pair slots of a window group's centre-of-mass pass held at a time (all windows of all pairs of a
-// batch of chains: 256 chains of N = 256, M = 128 in FP32 take 0.5 GiB).
+// Pair slots of a window group held at a time: for every pair of a batch of chains the C of each
+// centre-of-mass window, or (they share the memory) a value and a partner of each staging window, the
+// larger of the two: 24 values a pair for M = 128, ell = 8 in FP32, 0.75 GiB for 256 chains of N = 256.
 constexpr size_t kPairBytes = (size_t)4 << 30;
 
 // The stream of window group g.

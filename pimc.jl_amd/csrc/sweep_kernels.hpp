@@ -1122,13 +1122,6 @@ template <typename T, int DIM> __device__ __forceinline__ T pair_mult(const T *a
     return T(mm);
 }
 
-template <typename T, int DIM, bool CELLS, typename PathT>
-__device__ __forceinline__ T link_sum(const PathT &path, const Cells &C, int N, int nbins, const Prm<T> &P, int n,
-                                      int j, const T *pj, const T *pj1)
-{
-    return link_part<T, DIM, CELLS>(path, C, N, nbins, P, n, j, pj, pj1, 0, 1);
-}
-
 // The hard-sphere test of hardspherelevy! and move_polymer! (src/updates/
 // helper.jl:166-170, 385-389): whether the nearest bead at slice j among the
 // stencil candidates of q (find_nn), other than particle n's, is closer than

@@ -160,13 +160,11 @@ template <typename T, int DIM> __device__ __forceinline__ T dist2_min(const T *x
 // --- ordered pair lists of a chunk of particles ---
 
 // LDS layout of the chunk machinery: candidate masks (kChunk x nq words),
-// counts, offsets, ends of the earlier partners, per-try sums, then the slot
-// pool (partner index with the hit flag in bit 15, owner, nval values: with
-// one value, pa and pc name the same array).
+// counts, offsets, then the slots (partner index and owner).
 struct ChunkLds {
-    size_t mask, cnt, off, nb, spec, misc, pq, po, pa, pc, end;
+    size_t mask, cnt, off, misc, pq, po, end;
 };
-__host__ __device__ inline ChunkLds chunk_lds(size_t o, int N, int cap, int tsize, int nval)
+__host__ __device__ inline ChunkLds chunk_lds(size_t o, int N, int cap)
 {
     ChunkLds L;
     const int nq = (N + 63) / 64;
@@ -175,41 +173,25 @@ __host__ __device__ inline ChunkLds chunk_lds(size_t o, int N, int cap, int tsiz
     L.cnt = o;
     o = align16(o + kChunk * 4);
     L.off = o;
-    o = align16(o + (kChunk + 1) * 4);
-    L.nb = o;
     o = align16(o + kChunk * 4);
-    L.spec = o;
-    o = align16(o + kChunk * 8);
     L.misc = o;
     o = align16(o + 16);
     L.pq = o;
     o = align16(o + (size_t)cap * 2);
     L.po = o;
-    o = align16(o + (size_t)cap);
-    L.pa = o;
-    o = align16(o + (size_t)cap * tsize);
-    L.pc = L.pa; // one value per slot: pa and pc are the same array
-    if (nval > 1) {
-        L.pc = o;
-        o = align16(o + (size_t)cap * tsize);
-    }
-    L.end = o;
+    L.end = align16(o + (size_t)cap);
     return L;
 }
 
-template <typename T> struct ChunkPtr {
+struct ChunkPtr {
     unsigned long long *mask;
-    int *cnt, *off, *nb, *misc;
-    double *spec;
+    int *cnt, *off, *misc;
     unsigned short *pq;
     unsigned char *po;
-    T *pa, *pc;
     __device__ __forceinline__ ChunkPtr(unsigned char *s, const ChunkLds &L)
         : mask(reinterpret_cast<unsigned long long *>(s + L.mask)), cnt(reinterpret_cast<int *>(s + L.cnt)),
-          off(reinterpret_cast<int *>(s + L.off)), nb(reinterpret_cast<int *>(s + L.nb)),
-          misc(reinterpret_cast<int *>(s + L.misc)), spec(reinterpret_cast<double *>(s + L.spec)),
-          pq(reinterpret_cast<unsigned short *>(s + L.pq)), po(s + L.po), pa(reinterpret_cast<T *>(s + L.pa)),
-          pc(reinterpret_cast<T *>(s + L.pc))
+          off(reinterpret_cast<int *>(s + L.off)), misc(reinterpret_cast<int *>(s + L.misc)),
+          pq(reinterpret_cast<unsigned short *>(s + L.pq)), po(s + L.po)
     {
     }
 };
@@ -340,8 +322,8 @@ template <int DIM, typename Visit> __device__ __forceinline__ void grid_visit(co
 // each the partners q with cand(p, q), by index.  Fills as many particles as
 // the pool holds (at least one: cap >= N).  Returns the number of particles filled (0: a caller's
 // loop over the particles has to end); X.misc[1] is the slot count.  All threads of the workgroup.
-template <int DIM = 2, typename T, typename Cand>
-__device__ inline int chunk_slots(ChunkPtr<T> &X, int pa, int N, int cap, int kc, Cand cand,
+template <int DIM = 2, typename Cand>
+__device__ inline int chunk_slots(ChunkPtr &X, int pa, int N, int cap, int kc, Cand cand,
                                   const WinGrid *G = nullptr)
 {
     const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nwv = nt >> 6;
@@ -481,7 +463,7 @@ __host__ __device__ __forceinline__ size_t pair_row(int p) { return (size_t)p * 
 
 // Buffers of the centre-of-mass kernels.  Per particle (window chains only, by
 // part_base) wbnd[. * nwin + w] bounds its old beads in window w, rbnd its old
-// ring, shift/unif hold its try, cnt the listed partners; per pair slot
+// ring, shift its try's displacement, cnt the listed partners; per pair slot
 // (ChainDev::pair_off + pair_row(p) + k, the k-th listed partner of p by index)
 // partner; per window and slot (at nval times the chain's pair offset)
 // cval: C of the window, with +0 for "no term within the cut-off" (a value of
@@ -585,8 +567,17 @@ inline int stage_budget(int N, int ell, int dim, int tsize)
     take((size_t)N * tsize);
     take((size_t)N);
     o = grid_lds(o, N, dim).end;
+    take((size_t)kChunk * ((N + 63) / 64) * 8);
+    for (int bytes : {kChunk * 4, (kChunk + 1) * 4, kChunk * 4, kChunk * 8, 16}) take((size_t)bytes);
     const size_t fixed = o;
-    auto bytes = [&](int cap) { return chunk_lds(fixed, N, cap, tsize, 2).end; };
+    auto bytes = [&](int cap) { // per pair: partner, owner, two values
+        o = fixed;
+        take((size_t)cap * 2);
+        take((size_t)cap);
+        take((size_t)cap * tsize);
+        take((size_t)cap * tsize);
+        return o;
+    };
     int cap = std::min(8192, kChunk * std::max(1, N - 1));
     while (cap > N && bytes(cap) > 64 * 1024) cap -= 64;
     return std::max(cap, N);
@@ -1379,7 +1370,6 @@ __global__ void __launch_bounds__(1024) k_com_dec(SweepArgs a, ComBuf<T> B, int 
         if (tid == 0) atomicOr(a.status + c, 2);
         return;
     }
-    const Prm<T> P = reinterpret_cast<const Prm<T> *>(a.prm)[c];
     const ComDecLds L = com_dec_lds(N, (int)sizeof(T), cap);
     double *const s_spec = reinterpret_cast<double *>(smem + L.spec);
     T *const su = reinterpret_cast<T *>(smem + L.su);
@@ -1513,7 +1503,7 @@ __host__ __device__ inline MeasWinLds meas_win_lds(int N, int lc, int dim, int t
     L.bnd = o;
     o = align16(o + (size_t)N * 16);
     L.gr = grid_lds(o, N, dim);
-    L.ck = chunk_lds(L.gr.end, N, cap, tsize, 1);
+    L.ck = chunk_lds(L.gr.end, N, cap);
     return L;
 }
 
@@ -1584,7 +1574,7 @@ template <typename T, int DIM> __global__ void __launch_bounds__(512) k_meas_win
     const MeasWinLds L = meas_win_lds(N, lc, DIM, (int)sizeof(T), cap);
     T *ob = reinterpret_cast<T *>(smem + L.ob);
     float4 *bnd = reinterpret_cast<float4 *>(smem + L.bnd);
-    ChunkPtr<T> X(smem, L.ck);
+    ChunkPtr X(smem, L.ck);
     const T *const gpath = reinterpret_cast<const T *>(a.pos) + ch.pos_off;
     for (int t = 0; t <= m; ++t) {
         const int j = (s0 + t) % M;
