@@ -592,8 +592,8 @@ inline int stage_budget(int N, int ell, int dim, int tsize)
 // keep = 0) sets the largest chain, so arrays that are not in use together share
 // their place: the A values follow the row masks, the decisions the column masks,
 // a row's end in the pair list is the fourth word of its particle's bound, and a
-// pair's row waits in the place of its C.  2D FP32, ell = 8: N <= 922; 868 with a
-// place each.
+// pair's row waits in the place of its C.  2D FP32, ell = 8: N <= 922 (868 with a
+// place each, 914 on the pair slots per chunk).
 struct StageLds {
     size_t ob, nb, bnd, sp, ncand, cmask, coff, misc, pa, pq, pc, end;
     GridLds gr;
@@ -666,8 +666,8 @@ template <typename T> struct StagePairs {
 // work (four pairings a slice); two workgroups share a CU, so one's decisions,
 // a serial chain, run beside the other's pairs.  Against pair slots per chunk of 64
 // tries, each pair from both sides (six pairings): 16 measuring sweeps of 256 chains
-// of N = 256, M = 128, FP32, 45.2 -> 40.0 ms; 64 chains of N = 400, M = 512, whose
-// blocks fill a CU alone, stay at 65 to 67 ms.
+// of N = 256, M = 128, FP32, 45.2 -> 40.0 ms; 64 chains of N = 400, M = 512 stayed at 67 ms
+// while their blocks took a CU alone and take 61 ms since two fit (StageLds).
 template <typename T, int DIM>
 __global__ void __launch_bounds__(1024) k_stage_win(SweepArgs a, ComBuf<T> B, int R, int cap, int keep, int budget)
 {
