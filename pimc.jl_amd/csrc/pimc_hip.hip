@@ -728,9 +728,10 @@ template <typename T, int DIM> void launch_win_d(pimc_ctx *c, const SweepArgs &b
         hipLaunchKernelGGL((k_stage_win<T, DIM>), dim3((unsigned)c->win_seg, (unsigned)nb), dim3(c->nt_stage),
                            c->lds_stage, st, v, B, c->rows_stage, c->cap_stage, c->keep_stage, c->stage_cand);
         HIPCHK(hipGetLastError());
-        hipLaunchKernelGGL((k_com_bounds<T, DIM>), dim3(blk, (unsigned)nb), dim3(256), c->lds_cbnd, st, v, B);
+        hipLaunchKernelGGL((k_com_bounds<T, DIM>), dim3(blk, (unsigned)nb), dim3(64 * std::min(16, c->spec_nwin)),
+                           c->lds_cbnd, st, v, B);
         HIPCHK(hipGetLastError());
-        hipLaunchKernelGGL((k_com_pairs<T, DIM>), dim3(blk, (unsigned)nb), dim3(256), 0, st, v, B);
+        hipLaunchKernelGGL((k_com_pairs<T, DIM>), dim3(blk, (unsigned)nb), dim3(1024), 0, st, v, B);
         HIPCHK(hipGetLastError());
         hipLaunchKernelGGL((k_com_spec<T, DIM>), dim3((unsigned)c->spec_nwin, (unsigned)nb), dim3(c->nt_cspec),
                            c->lds_cspec, st, v, B, c->rows_cspec, c->cap_cspec);

@@ -997,11 +997,13 @@ __device__ __forceinline__ bool com_near(float4 A, const T *da, float4 B, const 
 constexpr int kBndPart = 64; // particles per workgroup of k_com_bounds
 
 // The tries' shifts and the bounds of the old beads: grid (particle blocks,
-// chains), 256 threads, four windows of 64 particles at a time (the particles of
-// a slice are consecutive in memory).  A window's bound: the middle of the beads'
+// chains), one wave per window of 64 particles (the particles of a slice are
+// consecutive in memory), up to 16 waves: a bound is a chain of dependent loads.
+// With 4 waves a workgroup 64 chains of N = 400, M = 256 took 121 us, sparse chains
+// of N = 97, M = 128 39 us of a sweep of 390.  A window's bound: the middle of the beads'
 // extent, and the largest distance from it; a ring's: the same of its windows'
 // bounds, unwrapped against window 0's.
-template <typename T, int DIM> __global__ void __launch_bounds__(256) k_com_bounds(SweepArgs a, ComBuf<T> B)
+template <typename T, int DIM> __global__ void __launch_bounds__(1024) k_com_bounds(SweepArgs a, ComBuf<T> B)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const int c = a.whole[blockIdx.y];
@@ -1015,7 +1017,7 @@ template <typename T, int DIM> __global__ void __launch_bounds__(256) k_com_boun
     float4 *s_b = reinterpret_cast<float4 *>(smem); // [window][64]
     const T *const gpath = reinterpret_cast<const T *>(a.pos) + ch.pos_off;
     const size_t part = (size_t)ch.part_base + p;
-    for (int w = threadIdx.x >> 6; w < nw; w += 4) {
+    for (int w = threadIdx.x >> 6; w < nw; w += (int)blockDim.x >> 6) {
         if (p >= N) continue;
         const int s0 = w * lc, m = min(lc, M - s0);
         T r0[DIM];
@@ -1084,8 +1086,8 @@ template <typename T, int DIM> __global__ void __launch_bounds__(256) k_com_boun
 }
 
 // The listed partners q < p of each particle, by index: grid (blocks of 64
-// particles, chains), 256 threads, one wave per particle and 64 partners at a time.
-template <typename T, int DIM> __global__ void __launch_bounds__(256) k_com_pairs(SweepArgs a, ComBuf<T> B)
+// particles, chains), one wave per particle and 64 partners at a time, 16 waves.
+template <typename T, int DIM> __global__ void __launch_bounds__(1024) k_com_pairs(SweepArgs a, ComBuf<T> B)
 {
     const int c = a.whole[blockIdx.y];
     const ChainDev ch = a.chains[c];
@@ -1095,7 +1097,7 @@ template <typename T, int DIM> __global__ void __launch_bounds__(256) k_com_pair
     const float4 *rb = B.rbnd + ch.part_base;
     const T *sd = B.shift + (size_t)ch.part_base * 2;
     const int p1 = min(N, ((int)blockIdx.x + 1) * 64);
-    for (int p = (int)blockIdx.x * 64 + (threadIdx.x >> 6); p < p1; p += 4) {
+    for (int p = (int)blockIdx.x * 64 + (threadIdx.x >> 6); p < p1; p += (int)blockDim.x >> 6) {
         unsigned short *row = B.row(ch, p);
         const float4 A = rb[p];
         const T da[2] = {sd[p * 2], DIM > 1 ? sd[p * 2 + 1] : T(0)};
