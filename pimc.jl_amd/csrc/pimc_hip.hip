@@ -1432,7 +1432,13 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
             int maxM = 1;
             for (int id : c->whole_lds_ids) {
                 const ChainDev &h = c->ch[id];
-                const bool fits = h.M <= kAllPairsMaxM &&
+                // A short FP32 ring leaves most of a wave's lanes idle there, where k_sweep_whole has all of them on
+                // links and particles, and is the faster one.  k_sweep_whole / k_sweep_allpairs, ms a sweep: 2D, 1000
+                // chains, M = 16, N = 12 0.379 / 0.368, N = 16 0.490 / 0.511, N = 30 0.933 / 1.011, N = 60 2.190 / 2.274; M = 17,
+                // N = 30 1.025 / 1.011.  1D, where a pair is half the work, 512 chains, N = 30: M = 32 0.429 / 0.483, M = 48
+                // 0.458 / 0.483, M = 64 0.507 / 0.477.  In FP64 it is 1.01 to 2.1 times as fast here from M = 8 on
+                const bool lanes = ts == 8 || (h.dim == 1 ? h.M > 48 : h.M > 16 || h.N <= 12);
+                const bool fits = lanes && h.M <= kAllPairsMaxM &&
                                   allpairs_lds(h.N, h.M, h.dim, ts, allpairs_groups(h.M)).end <= 159 * 1024; // and 1 KiB static
                 if (h.pair == kPairGaussian && h.pair_in_accept && h.swaps == 0 && h.nbins >= 3 && fits) {
                     c->allpairs_ids.push_back(id);

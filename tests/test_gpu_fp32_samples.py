@@ -53,6 +53,12 @@ def test_small_pair_chains(N, M, ell):
     check(N, M, ell, 3.0, 3)
 
 
+@pytest.mark.parametrize("N,M,ell,dim", [(12, 16, 8, 2), (13, 16, 8, 2), (13, 17, 8, 2), (30, 48, 8, 1), (30, 49, 8, 1)])
+def test_small_pair_chains_at_the_kernels_border(N, M, ell, dim):
+    """Short rings run on k_sweep_whole, the next longer ones on k_sweep_allpairs."""
+    check(N, M, ell, 3.0, 3, dim=dim)
+
+
 @pytest.mark.parametrize("N,M,ell,L,nbins,dim", [(65, 12, 5, 6.0, 6, 2), (150, 8, 8, 3.0, 3, 2), (260, 8, 4, 4.0, 4, 2),
                                                  (200, 12, 12, 3.0, 3, 2), (400, 40, 8, 10.0, 10, 2), (110, 16, 8, 20.0, 12, 1),
                                                  (290, 36, 32, 6.0, 6, 2)])
