@@ -116,6 +116,13 @@ struct pimc_ctx {
     size_t lds_allpairs = 0, lds_apmeas = 0;
     int apmeas_nblk = 1;
     double *d_apmeas_part = nullptr;   // their split estimators' partial sums [id][window][6]
+    // Where the chains run whole are spread over several of k_sweep_whole, k_sweep_ideal and
+    // k_sweep_allpairs, the latter two (ideal_beside: k_sweep_ideal only) run beside the other on a stream
+    // of their own, forked from stream and joined back into it at each launch: a kernel of few or long
+    // chains does not fill the chip.  Chains share no buffer
+    hipStream_t beside = nullptr;
+    hipEvent_t ev_beside[2] = {nullptr, nullptr};
+    bool ideal_beside = false;
     // Gaussian-pair chains on the window staging and centre-of-mass kernels, with and without
     // cell lists for the estimators (index 0: cells, 1: all-pairs); win_all: both
     std::vector<int> win_ids[2], win_all;
@@ -308,31 +315,36 @@ void launch_whole_t(pimc_ctx *c, SweepArgs a, const std::vector<int> &all, int l
     HIPCHK(hipGetLastError());
 }
 
-template <typename T, int DIM> void launch_ideal_t(pimc_ctx *c, SweepArgs a)
+template <typename T, int DIM> void launch_ideal_t(pimc_ctx *c, SweepArgs a, hipStream_t st)
 {
     if (c->ideal_ids.empty()) return;
     a.whole = c->d_ideal;
     auto k = k_sweep_ideal<T, DIM>;
     if (c->lds_ideal > 65536) HIPCHK(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->lds_ideal));
-    hipLaunchKernelGGL(k, dim3((unsigned)c->ideal_ids.size()), dim3(kIdealThreads), c->lds_ideal, c->stream, a);
+    hipLaunchKernelGGL(k, dim3((unsigned)c->ideal_ids.size()), dim3(kIdealThreads), c->lds_ideal, st, a);
     HIPCHK(hipGetLastError());
 }
 
-template <typename T, int DIM> void launch_allpairs_t(pimc_ctx *c, SweepArgs a)
+template <typename T, int DIM> void launch_allpairs_t(pimc_ctx *c, SweepArgs a, hipStream_t st)
 {
     if (c->allpairs_ids.empty()) return;
     a.whole = c->d_allpairs;
     a.link_group = c->allpairs_g;
     auto k = k_sweep_allpairs<T, DIM>;
     if (c->lds_allpairs > 65536) HIPCHK(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->lds_allpairs));
-    hipLaunchKernelGGL(k, dim3((unsigned)c->allpairs_ids.size()), dim3(kAllPairsThreads), c->lds_allpairs, c->stream, a);
+    hipLaunchKernelGGL(k, dim3((unsigned)c->allpairs_ids.size()), dim3(kAllPairsThreads), c->lds_allpairs, st, a);
     HIPCHK(hipGetLastError());
 }
 
 template <typename T, int DIM> void launch_whole_d(pimc_ctx *c, const SweepArgs &a)
 {
-    launch_ideal_t<T, DIM>(c, a);
-    launch_allpairs_t<T, DIM>(c, a);
+    const hipStream_t side = c->beside ? c->beside : c->stream;
+    if (c->beside) {
+        HIPCHK(hipEventRecord(c->ev_beside[0], c->stream));
+        HIPCHK(hipStreamWaitEvent(side, c->ev_beside[0], 0));
+    }
+    launch_ideal_t<T, DIM>(c, a, side);
+    launch_allpairs_t<T, DIM>(c, a, c->ideal_beside ? c->stream : side);
     const auto &wc = c->whole_cells_ids, &wb = c->whole_brute_ids, &wl = c->whole_lds_ids;
     // per list: analytic pairs, then tabulated-propagator chains, then those with swap moves
     launch_whole_t<T, DIM, true, false, false>(c, a, wc, 0, c->cells_tab0, c->d_whole_cells);
@@ -344,6 +356,10 @@ template <typename T, int DIM> void launch_whole_d(pimc_ctx *c, const SweepArgs 
     launch_whole_t<T, DIM, false, true, false>(c, a, wl, 0, c->lds_tab0, c->d_whole_lds);
     launch_whole_t<T, DIM, false, true, true>(c, a, wl, c->lds_tab0, c->lds_tperm0, c->d_whole_lds);
     launch_whole_t<T, DIM, false, true, true, true>(c, a, wl, c->lds_tperm0, (int)wl.size(), c->d_whole_lds);
+    if (c->beside) {
+        HIPCHK(hipEventRecord(c->ev_beside[1], side));
+        HIPCHK(hipStreamWaitEvent(c->stream, c->ev_beside[1], 0));
+    }
 }
 
 void launch_whole(pimc_ctx *c, const SweepArgs &a)
@@ -1456,6 +1472,19 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
                 c->apmeas_nblk = std::max(c->apmeas_nblk, (h.M + kMeasSlices - 1) / kMeasSlices);
             }
         }
+        // kernels beside each other where the chains are spread over several, ms a sweep on k_sweep_whole alone /
+        // one after the other / beside: 3 trapped pair chains of each N = 8..95, M = 256 5.45 / 6.69 / 5.47; 128 chains of
+        // N = 60, M = 100 and 128 with the pair action dropped 1.28 / 1.43 / 0.87 (measuring); 128 ideal and 128
+        // interacting swap chains of N = 20, M = 100 0.276 / 0.303 / 0.271
+        {
+            const bool whole = !(c->whole_cells_ids.empty() && c->whole_brute_ids.empty() && c->whole_lds_ids.empty());
+            const bool ideal = !c->ideal_ids.empty(), pairs = !c->allpairs_ids.empty();
+            c->ideal_beside = ideal && pairs && !whole;
+            if (c->ideal_beside || (whole && (ideal || pairs))) {
+                HIPCHK(hipStreamCreateWithFlags(&c->beside, hipStreamNonBlocking));
+                for (hipEvent_t &e : c->ev_beside) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            }
+        }
         // tabulated-propagator chains last in each list (their own kernel instantiation)
         {
             auto part = [&](std::vector<int> &v) {
@@ -1739,7 +1768,8 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
 int pimc_destroy(pimc_ctx *c)
 {
     if (!c) return PIMC_OK;
-    if (c->stream) (void)hipStreamSynchronize(c->stream);
+    for (hipStream_t st : {c->stream, c->stream2, c->beside})
+        if (st) (void)hipStreamSynchronize(st);
     drop_graphs(c);
     dfree(c->d_rs);
     void *ptrs[] = {c->d_ch, c->d_prm, c->d_tiles, c->d_pchain, c->d_pidx, c->d_pos, c->d_part_acc, c->d_placc, c->d_pcacc,
@@ -1761,6 +1791,9 @@ int pimc_destroy(pimc_ctx *c)
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
     if (c->ev_join) (void)hipEventDestroy(c->ev_join);
     if (c->stream2) (void)hipStreamDestroy(c->stream2);
+    for (hipEvent_t e : c->ev_beside)
+        if (e) (void)hipEventDestroy(e);
+    if (c->beside) (void)hipStreamDestroy(c->beside);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return PIMC_OK;
