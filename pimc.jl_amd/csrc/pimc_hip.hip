@@ -1657,8 +1657,8 @@ int pimc_create(pimc_ctx **out, const pimc_chain_desc *chains, int32_t n_chains,
             // window chains fill at most half of the CUs (one decision workgroup a chain: with
             // more, the decision kernels already occupy the chip and a second group only contends
             // for it).  One group against two, 16 measuring sweeps FP32: 64 chains of N = 400, M = 512
-            // 63.6 / 61.2 ms; 8 sweeps: 36 of N = 400, M = 400 13.3 / 12.9, 100 of N = 300, M = 100 even,
-            // but 4 of N = 97, M = 32, which launches bound, 1.75 / 2.12
+            // 61.5 / 60.5 ms; 8 sweeps: 36 of N = 400, M = 400 12.7 / 11.9, 100 of N = 300, M = 100 9.98 / 9.87,
+            // but 4 of N = 97, M = 32, which launches bound, 1.70 / 2.06
             const int nwc = (int)c->win_all.size();
             const bool two = nwc >= 2 && 2 * nwc <= cu;
             int split = nwc;
